@@ -7,18 +7,18 @@
 // ::F32 keeps Q and output in f32.
 //
 // Design for MI355X (dense contraction on the matrix cores):
-//   * workgroup = 4 wave64 sharing one KV head: the HW (<= 4) query heads of a GQA group times
-//     32 * 4 / HW query tokens; every wave owns 32 queries of one head, so the 4 waves of a
-//     G = 4 group read each K/V tile from LDS once per head instead of from HBM;
+//   * a workgroup serves one KV head: the HW (<= 4) query heads of a GQA group times 32 * 4 / HW
+//     query tokens, in 4 column blocks of 32 queries of one head, one wave each (8-wave kernels:
+//     two key groups of 4), so the 4 waves of a G = 4 group read each K/V tile from LDS once
+//     per head instead of from HBM;
 //   * S^T = K Q^T and O^T = V^T P^T with v_mfma_f32_32x32x16_f16: the S^T accumulator layout
 //     (lane = query column, 16 keys per lane) is exactly the B-operand layout P^T needs, so P
-//     never goes through LDS; K is read from LDS row-major, V is stored transposed in LDS
-//     (d-major) so each A operand is two ds_read_b64;
-//   * 64-key K/V tiles, global loads for tile i+1 issued before the MFMAs of tile i;
-//   * causal skipping per wave (32-key sub-blocks past its last query are not computed) and
-//     masking only on sub-blocks that cross the diagonal; heaviest query tiles dispatch first
-//     (flash_attention.metal:202-205) and the head-group index varies fastest so the 8 KV heads
-//     spread over the 8 XCDs (each XCD's L2 keeps its head's K/V);
+//     never goes through LDS; K and V sit row-major in LDS (16-byte chunks swizzled), K read by
+//     ds_read_b128, V transposed by ds_read_b64_tr_b16;
+//   * the next tile's global loads issued before the MFMAs of the current one;
+//   * causal skipping per wave and masking only on tiles that cross the diagonal; heaviest query
+//     tiles dispatch first (flash_attention.metal:202-205) and the head-group index varies
+//     fastest so the 8 KV heads spread over the 8 XCDs (each XCD's L2 keeps its head's K/V);
 //   * values that f16 cannot hold exactly (f32 and q8_0 caches, f32 Q, f32 P) are split as
 //     x = hi + lo with hi = f16(x), lo = f16(x - hi) and contracted with extra MFMAs
 //     (hi*hi + hi*lo + lo*hi), which keeps ~22 significant bits;
@@ -42,8 +42,6 @@ typedef __attribute__((address_space(3))) v4s lds_v4s;
 
 constexpr int kThreads = 256;
 constexpr int kTile = 64;       // keys per LDS tile
-constexpr int kKStr = 136;      // K row stride in halves (128 + 8 pad)
-constexpr int kVStr = 72;       // V^T row stride in halves (64 + 8 pad)
 
 struct PrefillArgs {
     const float* q;
@@ -190,6 +188,11 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// lds_barrier as one asm, which also keeps the compiler from moving memory accesses across it.
+__device__ __forceinline__ void lds_sync() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // x is materialised as one f32 value for both halves (see as_f32): a product folded into a
 // single-rounding conversion for hi alone would leave hi + lo one f16 ulp off at f16 ties.
 __device__ __forceinline__ void split_f16(float x, uint16_t& hi, uint16_t& lo) {
@@ -201,12 +204,6 @@ __device__ __forceinline__ void split_f16(float x, uint16_t& hi, uint16_t& lo) {
 __device__ __forceinline__ half8 lds_b128(const uint16_t* p) {
     return __builtin_bit_cast(half8, *reinterpret_cast<const uint4*>(p));
 }
-__device__ __forceinline__ half8 lds_2xb64(const uint16_t* p0, const uint16_t* p1) {
-    uint2 a = *reinterpret_cast<const uint2*>(p0);
-    uint2 b = *reinterpret_cast<const uint2*>(p1);
-    uint4 c = make_uint4(a.x, a.y, b.x, b.y);
-    return __builtin_bit_cast(half8, c);
-}
 __device__ __forceinline__ half8 pack8(const uint16_t (&x)[8]) {
     uint4 c;
     c.x = x[0] | ((uint32_t)x[1] << 16);
@@ -214,6 +211,32 @@ __device__ __forceinline__ half8 pack8(const uint16_t (&x)[8]) {
     c.z = x[4] | ((uint32_t)x[5] << 16);
     c.w = x[6] | ((uint32_t)x[7] << 16);
     return __builtin_bit_cast(half8, c);
+}
+
+// x = hi + lo (split_f16) for 8 values: the conversions in pairs, and the residual x - hi by one
+// exact fma with the f16 operand. Callers pass products through as_f32.
+__device__ __forceinline__ void split8(const float (&x)[8], half8& hi, half8& lo) {
+    typedef _Float16 hf2 __attribute__((ext_vector_type(2)));
+    typedef float ff2 __attribute__((ext_vector_type(2)));
+    uint32_t hw[4], lw[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const ff2 v = {x[2 * i], x[2 * i + 1]};
+        const hf2 h = __builtin_convertvector(v, hf2);
+        const ff2 r = {fmaf((float)h.x, -1.0f, v.x), fmaf((float)h.y, -1.0f, v.y)};
+        hw[i] = __builtin_bit_cast(uint32_t, h);
+        lw[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, hf2));
+    }
+    hi = __builtin_bit_cast(half8, u32x4{hw[0], hw[1], hw[2], hw[3]});
+    lo = __builtin_bit_cast(half8, u32x4{lw[0], lw[1], lw[2], lw[3]});
+}
+
+// V^T operand of one 16-key step: this lane's 8 keys of one dim from two transposed reads of the
+// row-major tile (rows r and r + 8 of 256 bytes)
+__device__ __forceinline__ half8 v_operand(const uint8_t* p) {
+    const v4s lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)p);
+    const v4s hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p + 8 * 256));
+    return __builtin_bit_cast(half8, __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
 // value combined with that of lane l ^ 32 (v_permlane32_swap: VALU, no LDS round trip)
@@ -319,232 +342,11 @@ __device__ __forceinline__ void q_convert_half(const u32x4 (&raw)[8], float scal
     }
 }
 
-// KV = cache type; HW = query heads per workgroup (1, 2, 4); QS = split Q (F32 precision);
-// PS = split P; OF32 = f32 output.
-template <int KV, int HW, bool QS, bool PS, bool OF32>
-__global__ void __launch_bounds__(kThreads, 2)
-prefill_kernel(PrefillArgs a) {
-    if (a.gate && *a.gate != a.tag) return;  // the fast launch before this one was exact
-    constexpr bool KS = (KV != BRASA_KV_F16);  // cache values need hi/lo
-    constexpr int NK = KS ? 2 : 1;
-    constexpr int TPW = 32 * 4 / HW;            // query tokens per workgroup
-    constexpr int RB = KvTraits<KV>::row_bytes;
-
-    __shared__ __attribute__((aligned(16))) uint16_t s_k[NK][kTile * kKStr];
-    __shared__ __attribute__((aligned(16))) uint16_t s_vt[NK][kDim * kVStr];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int col = lane & 31;       // query column of the MFMA tiles
-    const int u = lane >> 5;         // lane half
-
-    const int hg = blockIdx.x;                            // head group (fastest: spreads XCDs)
-    const int tile = a.ntiles - 1 - (int)blockIdx.y;      // heaviest query tiles first
-    const int h = hg * HW + (wave % HW);
-    const int kh = (hg * HW) / a.group;
-    const int t0 = tile * TPW;
-    const int tw0 = t0 + 32 * (wave / HW);                // first query token of this wave
-    const int lk = a.pos0 + a.tokens;
-    const int kend_wg = a.pos0 + min(t0 + TPW, a.tokens);  // keys [0, kend_wg) are read
-    const int kend_w = a.pos0 + min(tw0 + 32, a.tokens);   // this wave needs [0, kend_w)
-
-    // ---- Q^T B-operands: k-step t holds d = 16t + 8u + j ------------------------------
-    const int tq = tw0 + col;
-    const bool qvalid = tq < a.tokens;
-    half8 qh[8], ql[QS ? 8 : 1];
-    {
-        const float* qrow = a.q + ((size_t)(qvalid ? tq : 0) * a.hq + h) * kDim;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const float4* p = reinterpret_cast<const float4*>(qrow + 16 * t + 8 * u);
-            float4 x0 = p[0], x1 = p[1];
-            float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-            uint16_t hi[8], lo[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float sx = qvalid ? as_f32(xs[j] * a.scale) : 0.0f;
-                if (QS) split_f16(sx, hi[j], lo[j]);
-                else hi[j] = f2h(sx);
-            }
-            qh[t] = pack8(hi);
-            if (QS) ql[t] = pack8(lo);
-        }
-    }
-
-    f32x16 acc[4];
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[dt][i] = 0.0f;
-    float m2 = -INFINITY;  // running max of s * log2(e)
-    float lsum = 0.0f;     // this lane's share of the softmax denominator
-    const int qabs = a.pos0 + tq;
-
-    // ---- global -> register staging of one 64-key tile ----------------------------------
-    // item i of thread (wave, lane): key = lane, 8-dim chunk = wave + 4 i (i = 0..3)
-    const size_t kstride = (size_t)a.hkv * RB;
-    const uint8_t* kbase = a.k + (size_t)kh * RB;
-    const uint8_t* vbase = a.v + (size_t)kh * RB;
-    Kv8<KV> rk[4], rv[4];
-    auto load_tile = [&](int kb) {
-        const size_t row = (size_t)(kb + lane) * kstride;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            rk[i].load(kbase + row, 8 * (wave + 4 * i));
-            rv[i].load(vbase + row, 8 * (wave + 4 * i));
-        }
-    };
-    auto store_tile = [&]() {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c8 = 8 * (wave + 4 * i);
-            float kf[8], vf[8];
-            rk[i].to_float(kf);
-            rv[i].to_float(vf);
-            const float ks = rk[i].scale(), vs = rv[i].scale();
-            uint16_t khi[8], klo[8], vhi[8], vlo[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (KS) {
-                    split_f16(KV == BRASA_KV_Q8_0 ? as_f32(kf[e] * ks) : kf[e], khi[e], klo[e]);
-                    split_f16(KV == BRASA_KV_Q8_0 ? as_f32(vf[e] * vs) : vf[e], vhi[e], vlo[e]);
-                } else {
-                    khi[e] = f2h(kf[e]);
-                    vhi[e] = f2h(vf[e]);
-                }
-            }
-            *reinterpret_cast<half8*>(&s_k[0][lane * kKStr + c8]) = pack8(khi);
-            if (KS) *reinterpret_cast<half8*>(&s_k[NK - 1][lane * kKStr + c8]) = pack8(klo);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                s_vt[0][(c8 + e) * kVStr + lane] = vhi[e];
-                if (KS) s_vt[NK - 1][(c8 + e) * kVStr + lane] = vlo[e];
-            }
-        }
-    };
-
-    load_tile(0);
-    for (int kb = 0; kb < kend_wg; kb += kTile) {
-        __syncthreads();  // previous tile fully consumed
-        store_tile();
-        __syncthreads();
-        if (kb + kTile < kend_wg) load_tile(kb + kTile);
-
-        if (kb >= kend_w) continue;  // this wave's queries are all before the tile
-        const int nsub = (kb + 32 < kend_w) ? 2 : 1;
-
-        // S^T for the two 32-key sub-blocks
-        f32x16 s[2];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s[b][i] = 0.0f;
-            if (b < nsub) {
-                const uint16_t* krow = &s_k[0][(32 * b + col) * kKStr + 8 * u];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const half8 ka = lds_b128(krow + 16 * t);
-                    s[b] = mfma(ka, qh[t], s[b]);
-                    if (QS) s[b] = mfma(ka, ql[t], s[b]);
-                    if (KS) {
-                        const half8 kl = lds_b128(&s_k[NK - 1][(32 * b + col) * kKStr + 8 * u + 16 * t]);
-                        s[b] = mfma(kl, qh[t], s[b]);
-                    }
-                }
-            }
-        }
-        // scale to log2 domain, causal mask, tile max
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int kb2 = kb + 32 * b;
-            const bool need_mask = (kb2 + 31 > a.pos0 + tw0) || (kb2 + 31 >= lk);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int key = kb2 + 8 * (i / 4) + 4 * u + (i % 4);
-                float x = s[b][i] * kLog2e;
-                if (b >= nsub || (need_mask && (key > qabs || key >= lk))) x = -INFINITY;
-                s[b][i] = x;
-                tmax = fmaxf(tmax, x);
-            }
-        }
-        tmax = max_xor32(tmax);
-        const float mn = fmaxf(m2, tmax);  // finite: key 0 is visible to every query
-        const float alpha = __builtin_amdgcn_exp2f(m2 - mn);
-        m2 = mn;
-        lsum *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
-
-        // P^T B-operands and O^T += V^T P^T
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            if (b >= nsub) break;
-#pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                uint16_t ph[8], pl[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float p = __builtin_amdgcn_exp2f(s[b][8 * st + j] - mn);
-                    lsum += p;
-                    if (PS) split_f16(p, ph[j], pl[j]);
-                    else ph[j] = f2h(p);
-                }
-                const half8 pb = pack8(ph);
-                half8 plb;
-                if (PS) plb = pack8(pl);
-                const int key0 = 32 * b + 16 * st + 4 * u;
-#pragma unroll
-                for (int dt = 0; dt < 4; ++dt) {
-                    const int d = 32 * dt + col;
-                    const half8 va = lds_2xb64(&s_vt[0][d * kVStr + key0], &s_vt[0][d * kVStr + key0 + 8]);
-                    acc[dt] = mfma(va, pb, acc[dt]);
-                    if (PS) acc[dt] = mfma(va, plb, acc[dt]);
-                    if (KS) {
-                        const half8 vl = lds_2xb64(&s_vt[NK - 1][d * kVStr + key0],
-                                                   &s_vt[NK - 1][d * kVStr + key0 + 8]);
-                        acc[dt] = mfma(vl, pb, acc[dt]);
-                    }
-                }
-            }
-        }
-    }
-
-    // ---- normalise and write O[t, h, d] --------------------------------------------------
-    const float L = sum_xor32(lsum);
-    if (!qvalid) return;
-    const float inv = 1.0f / L;
-    const size_t obase = ((size_t)tq * a.hq + h) * kDim;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int d = 32 * dt + 8 * g + 4 * u;
-            const float y0 = as_f32(acc[dt][4 * g] * inv), y1 = as_f32(acc[dt][4 * g + 1] * inv);
-            const float y2 = as_f32(acc[dt][4 * g + 2] * inv), y3 = as_f32(acc[dt][4 * g + 3] * inv);
-            if (OF32) {
-                *reinterpret_cast<float4*>(static_cast<float*>(a.o) + obase + d) =
-                    make_float4(y0, y1, y2, y3);
-            } else {
-                uint2 w;
-                w.x = (uint32_t)f2h(y0) | ((uint32_t)f2h(y1) << 16);
-                w.y = (uint32_t)f2h(y2) | ((uint32_t)f2h(y3) << 16);
-                *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.o) + obase + d) = w;
-            }
-        }
-    }
-}
-
-
 // ---- f16 cache, F16 / F16_PF32 precision: the hot path -------------------------------------
 //
-// Same work decomposition and MFMA formulation as prefill_kernel, with the K/V staging moved off
-// the vector ALUs: each 64-key stage is copied HBM -> LDS by global_load_lds_dwordx4 (raw f16
-// rows, 16-byte chunks XOR-swizzled so the operand reads are bank-conflict free), K A-operands
-// are ds_read_b128 of those rows and V^T A-operands are ds_read_tr16_b64 of the same row-major
-// tile. Two stages alternate so stage i + 1 streams in while stage i is contracted. The O
+// Each 64-key stage is copied HBM -> LDS by global_load_lds_dwordx4 (raw f16 rows, 16-byte chunks
+// XOR-swizzled so the operand reads are bank-conflict free), K A-operands are ds_read_b128 of
+// those rows and V^T A-operands are ds_read_tr16_b64 of the same row-major tile. Two stages alternate so stage i + 1 streams in while stage i is contracted. The O
 // accumulator is only rescaled when a column's running max grows by more than 2^8 (P then stays
 // below 256, well inside f16), and masking runs only on tiles that cross the diagonal.
 constexpr int kStageHalves = kTile * kDim;  // one 64 x 128 f16 tile
@@ -671,7 +473,7 @@ __device__ __forceinline__ void f16_pp_tile(const PrefillArgs& a, const int tile
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave >> 2;  // group g contracts the workgroup's tiles g, g + 2, g + 4, ...
-    const int qw = wave & 3;    // head and 32-query block, as in prefill_kernel
+    const int qw = wave & 3;    // head and 32-query block
     const int col = lane & 31;
     const int u = lane >> 5;
 
@@ -1626,6 +1428,305 @@ prefill_f16_kernel4s(PrefillArgs a) {
                  a.o, tw0, a.tokens, a.hq, h);
 }
 
+// One 8-dim chunk of a cache row as the staging threads hold it: loaded into registers one stage
+// ahead, then split into the f16 hi (and, unless the cache is f16, lo) halves the tiles hold.
+// Plain loads: the other query tiles of the head read the same rows.
+template <int KV> struct Chunk8;
+template <> struct Chunk8<BRASA_KV_F32> {
+    f32x4 a, b;
+    __device__ __forceinline__ void load(const uint8_t* row, int c) {
+        a = *reinterpret_cast<const f32x4*>(row + 32 * c);
+        b = *reinterpret_cast<const f32x4*>(row + 32 * c + 16);
+    }
+    __device__ __forceinline__ void split(half8& hi, half8& lo) const {
+        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        split8(x, hi, lo);
+    }
+};
+template <> struct Chunk8<BRASA_KV_F16> {
+    u32x4 raw;
+    __device__ __forceinline__ void load(const uint8_t* row, int c) {
+        raw = *reinterpret_cast<const u32x4*>(row + 16 * c);
+    }
+    __device__ __forceinline__ void split(half8& hi, half8&) const {
+        hi = __builtin_bit_cast(half8, raw);
+    }
+};
+template <> struct Chunk8<BRASA_KV_Q8_0> {
+    u32x2 raw;
+    uint32_t sc;
+    __device__ __forceinline__ void load(const uint8_t* row, int c) {
+        raw = *reinterpret_cast<const u32x2*>(row + 8 * c);  // rows are 8-byte aligned
+        sc = *reinterpret_cast<const uint16_t*>(row + 128 + 2 * (c >> 2));
+    }
+    __device__ __forceinline__ void split(half8& hi, half8& lo) const {
+        const float s = h2f((uint16_t)sc);
+        float x[8];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            x[b] = (float)(int8_t)(raw.x >> (8 * b)) * s;  // exact: 18 significant bits
+            x[4 + b] = (float)(int8_t)(raw.y >> (8 * b)) * s;
+        }
+        split8(x, hi, lo);
+    }
+};
+
+// Every precision and cache type the f16 kernels above do not take: the F32 precision, F16_PF32
+// on f32 and q8_0 caches, F16 on f32 caches. KV = cache type; HW = query heads per workgroup
+// (1, 2, 4); QS = split Q (F32 precision); PS = split P; OF32 = f32 output.
+//
+// Bound: the matrix cores, at one MFMA per kept product of the hi / lo splits (up to 3 for QK^T
+// and 3 for PV). Workgroup = 8 waves: 4 column blocks of 32 queries (heads x tokens, as the f16
+// kernels) times two key groups; group g contracts the 32-key stages g, g + 2, ... and the two
+// merge through LDS at the end, so a SIMD holds two waves also when the launch has only one
+// workgroup per CU. The four waves of a group load the next stage's rows into registers, split
+// each value once and write f16 hi and lo tiles in the swizzled layouts of the f16 kernels (K
+// read by ds_read_b128, V transposed by ds_read_b64_tr_b16): a value is split once per workgroup
+// and 32 x 4 queries instead of once per wave, and no transposed tile is written. Two stage
+// buffers per group, one barrier per stage: stage i + 1 is written while stage i is contracted.
+// Against the kernel before it (four waves, one 64-key stage buffer, V written transposed two
+// bytes at a time; 32 heads over 8): f32 cache, F32 precision, T = 1000 206 -> 49 us (39 -> 167
+// TFLOP/s of the 3x as many that the splits contract), T = 2000 402 -> 119 us; q8_0 cache,
+// F16_PF32, T = 600 89 -> 33 us; f16 cache, F32 precision, T = 600 57 -> 26 us.
+template <int KV, int HW, bool QS, bool PS, bool OF32>
+__global__ void __launch_bounds__(2 * kThreads, 1)
+prefill_split_kernel(PrefillArgs a) {
+    constexpr bool KS = KV != BRASA_KV_F16;  // cache values need hi / lo
+    constexpr int NK = KS ? 2 : 1;
+    constexpr int TPW = 32 * 4 / HW;         // query tokens per workgroup
+    constexpr int RB = KvTraits<KV>::row_bytes;
+    constexpr int kBuf = 2 * NK * kStageHalvesS;  // one stage: K hi, K lo, V hi, V lo
+    constexpr int kXchHalves = 4 * 17 * 64 * 8;   // the group merge's exchange
+    __shared__ __attribute__((aligned(16))) uint16_t s_kv[4 * kBuf > kXchHalves ? 4 * kBuf : kXchHalves];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = wave >> 2;
+    const int qw = wave & 3;
+    const int col = lane & 31;       // query column of the MFMA tiles
+    const int u = lane >> 5;         // lane half
+
+    const int hg = blockIdx.x;                            // head group (fastest: spreads XCDs)
+    const int tile = a.ntiles - 1 - (int)blockIdx.y;      // heaviest query tiles first
+    const int h = hg * HW + (qw % HW);
+    const int kh = (hg * HW) / a.group;
+    const int t0 = tile * TPW;
+    const int tw0 = t0 + 32 * (qw / HW);                  // first query token of this wave
+    const int lk = a.pos0 + a.tokens;
+    const int kend_wg = a.pos0 + min(t0 + TPW, a.tokens);  // keys [0, kend_wg) are read
+    const int kend_w = a.pos0 + min(tw0 + 32, a.tokens);   // this wave needs [0, kend_w)
+    const int nst = (kend_wg + kTileS - 1) / kTileS;       // 32-key stages
+    // launches of up to 64 keys: one group takes them all (a merge costs more than a stage)
+    const int ngrp = nst <= 2 ? 1 : 2;
+    if (grp >= ngrp) return;
+    const int ng = (nst - grp + ngrp - 1) / ngrp;          // this group's
+    auto stage_of = [&](int i) { return ngrp * i + grp; };
+
+    // ---- staging: thread (row r0, chunk ch) of the group takes rows r0 and r0 + 16 ------------
+    const size_t kstride = (size_t)a.hkv * RB;
+    const uint8_t* kbase = a.k + (size_t)kh * RB;
+    const uint8_t* vbase = a.v + (size_t)kh * RB;
+    const int r0 = (threadIdx.x & 255) >> 4, ch = threadIdx.x & 15;
+    Chunk8<KV> rk[2], rv[2];
+    auto load_rows = [&](int i) {
+        const size_t row = (size_t)(stage_of(i) * kTileS + r0) * kstride;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            rk[j].load(kbase + row + 16 * j * kstride, ch);
+            rv[j].load(vbase + row + 16 * j * kstride, ch);
+        }
+    };
+    auto write_rows = [&](int i) {
+        uint16_t* t = s_kv + (2 * grp + (i & 1)) * kBuf;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int row = r0 + 16 * j;
+            half8 hi, lo;
+            rk[j].split(hi, lo);
+            *reinterpret_cast<half8*>(t + row * kDim + 8 * kswz(row, ch)) = hi;
+            if (KS) *reinterpret_cast<half8*>(t + kStageHalvesS + row * kDim + 8 * kswz(row, ch)) = lo;
+            rv[j].split(hi, lo);
+            *reinterpret_cast<half8*>(t + NK * kStageHalvesS + row * kDim + 8 * vswz(row, ch)) = hi;
+            if (KS) *reinterpret_cast<half8*>(t + 3 * kStageHalvesS + row * kDim + 8 * vswz(row, ch)) = lo;
+        }
+    };
+    if (0 < ng) load_rows(0);
+
+    // ---- Q^T B-operands: k-step t holds d = 16 t + 8 u + j ------------------------------------
+    const int tq = tw0 + col;
+    const bool qvalid = tq < a.tokens;
+    half8 qh[8], ql[QS ? 8 : 1];
+    {
+        const float* qrow = a.q + ((size_t)(qvalid ? tq : 0) * a.hq + h) * kDim;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const f32x4* p = reinterpret_cast<const f32x4*>(qrow + 16 * t + 8 * u);
+            const f32x4 x0 = p[0], x1 = p[1];
+            const float sc = qvalid ? a.scale : 0.0f;
+            const float xs[8] = {as_f32(x0.x * sc), as_f32(x0.y * sc), as_f32(x0.z * sc),
+                                 as_f32(x0.w * sc), as_f32(x1.x * sc), as_f32(x1.y * sc),
+                                 as_f32(x1.z * sc), as_f32(x1.w * sc)};
+            half8 lo;
+            split8(xs, qh[t], lo);
+            if (QS) ql[t] = lo;
+        }
+    }
+
+    // lane-constant byte offsets of the K operand rows and the V^T tr16 sources, as in
+    // prefill_f16_kernel4s
+    const uint32_t kcol = col * 256 + 16 * (u ^ (col & 1));
+    const int c14 = col & 14;
+    auto koff = [&](int t, int c) { return kcol + 16 * ((2 * t) ^ c); };
+    uint32_t voff[4];
+    {
+        const int sl = lane & 15, j = sl >> 2;
+        const int low = 2 * ((lane >> 4) & 1) + ((sl & 3) >> 1);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+            voff[dt] = (4 * u + j) * 256 + 16 * (4 * (dt ^ j) + low) + 8 * (sl & 1);
+    }
+
+    f32x16 acc[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[dt][i] = 0.0f;
+    float m_used = -INFINITY;  // shift of the column's exponentials (raw score units)
+    float lsum = 0.0f;         // this lane's share of the softmax denominator
+    const int qabs = a.pos0 + tq;
+    // rescale when the max grows by 2^8 in exp2 terms; at every growth where P is rounded to f16,
+    // which then holds each column's largest P exactly
+    const float kGrow = PS ? 8.0f / kLog2e : 0.0f;
+
+    auto scores = [&](int i, f32x16& s) {
+        const uint8_t* kt = reinterpret_cast<const uint8_t*>(s_kv + (2 * grp + (i & 1)) * kBuf);
+        int c = c14;
+        asm volatile("" : "+v"(c));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const half8 ka = lds_b128(reinterpret_cast<const uint16_t*>(kt + koff(t, c)));
+            s = mfma(ka, qh[t], s);
+            if (QS) s = mfma(ka, ql[t], s);
+            if (KS) {
+                const half8 kl = lds_b128(reinterpret_cast<const uint16_t*>(kt + koff(t, c)) + kStageHalvesS);
+                s = mfma(kl, qh[t], s);
+            }
+        }
+    };
+    auto contract = [&](int i, f32x16& s) {
+        const int kb = stage_of(i) * kTileS;
+        // causal mask (only on stages that reach past the wave's first query)
+        if ((kb + 31 > a.pos0 + tw0) || (kb + 31 >= lk)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = kb + 8 * (r / 4) + 4 * u + (r % 4);
+                s[r] = (key > qabs || key >= lk) ? -INFINITY : s[r];
+            }
+        }
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
+        tmax = max_xor32(tmax);
+        const bool grow = tmax > m_used + kGrow;
+        if (__builtin_amdgcn_ballot_w64(grow)) {
+            const float alpha = grow ? __builtin_amdgcn_exp2f((m_used - tmax) * kLog2e) : 1.0f;
+            if (grow) m_used = tmax;
+            lsum *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[dt][r] *= alpha;
+        }
+        // a column without a key so far has m = -inf and every s = -inf: P = 0
+        const float m = m_used == -INFINITY ? 0.0f : m_used;
+        const uint8_t* vt = reinterpret_cast<const uint8_t*>(s_kv + (2 * grp + (i & 1)) * kBuf + NK * kStageHalvesS);
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            float p[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                p[j] = __builtin_amdgcn_exp2f((s[8 * st + j] - m) * kLog2e);
+                lsum += p[j];
+            }
+            half8 pb, plb;
+            split8(p, pb, plb);
+            const int rows = 16 * st * 256;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                const half8 va = v_operand(vt + voff[dt] + rows);
+                acc[dt] = mfma(va, pb, acc[dt]);
+                if (PS) acc[dt] = mfma(va, plb, acc[dt]);
+                if (KS) acc[dt] = mfma(v_operand(vt + kStageHalvesS * 2 + voff[dt] + rows), pb, acc[dt]);
+            }
+        }
+    };
+
+    if (0 < ng) write_rows(0);
+    if (1 < ng) load_rows(1);
+    const int niter = (nst + ngrp - 1) / ngrp;  // group 0's stages: both groups pass the same barriers
+    for (int i = 0; i < niter; ++i) {
+        // stage i written by every wave of the group; its last reads of stage i - 1 returned
+        lds_sync();
+        const bool on = i < ng && stage_of(i) * kTileS < kend_w;
+        f32x16 s;
+        if (on) scores(i, s);
+        if (i + 1 < ng) {
+            write_rows(i + 1);
+            if (i + 2 < ng) load_rows(i + 2);
+        }
+        if (on) contract(i, s);
+    }
+    lds_sync();  // every stage read
+
+    // ---- merge the two groups' key halves: group 1 hands (m, l, O) to group 0 through LDS -----
+    // (17 16-byte chunks per lane, chunk-major: conflict-free 128-bit accesses)
+    f32x4* xch = reinterpret_cast<f32x4*>(s_kv) + qw * 17 * 64 + lane;
+    if (grp == 1) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+            xch[64 * c] = f32x4{acc[c >> 2][4 * (c & 3)], acc[c >> 2][4 * (c & 3) + 1],
+                                acc[c >> 2][4 * (c & 3) + 2], acc[c >> 2][4 * (c & 3) + 3]};
+        xch[64 * 16] = f32x4{m_used, lsum, 0.0f, 0.0f};
+    }
+    if (ngrp == 2) lds_sync();
+    if (grp == 1) return;
+    if (ngrp == 2) {
+        const f32x4 ml = xch[64 * 16];
+        const float M = fmaxf(m_used, ml[0]);  // finite: group 0 saw key 0
+        const float wa = __builtin_amdgcn_exp2f((m_used - M) * kLog2e);
+        const float wb = (ml[0] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((ml[0] - M) * kLog2e);
+        lsum = lsum * wa + ml[1] * wb;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const f32x4 o1 = xch[64 * c];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[c >> 2][4 * (c & 3) + j] = acc[c >> 2][4 * (c & 3) + j] * wa + o1[j] * wb;
+        }
+    }
+
+    // ---- normalise and write O[t, h, d] --------------------------------------------------
+    const float L = sum_xor32(lsum);
+    const float inv = 1.0f / L;  // padding columns: never stored
+    if constexpr (OF32) {
+        if (!qvalid) return;
+        const size_t obase = ((size_t)tq * a.hq + h) * kDim;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<f32x4*>(static_cast<float*>(a.o) + obase + 32 * dt + 8 * g + 4 * u) =
+                    f32x4{acc[dt][4 * g] * inv, acc[dt][4 * g + 1] * inv, acc[dt][4 * g + 2] * inv,
+                          acc[dt][4 * g + 3] * inv};
+    } else {
+        // this wave's own 17 KB of the exchange area (its merge has read them): 8 KB of rows
+        store_o_rows(acc, inv, reinterpret_cast<uint8_t*>(s_kv) + qw * 17 * 64 * 16, lane, a.o, tw0,
+                     a.tokens, a.hq, h);
+    }
+}
+
 // Kernel choice by workgroup count (one per query tile and head group), measured on one box at
 // hq 32 / hkv 8: up to two per CU the two-group kernel, which splits each tile's keys over two
 // wave groups (T = 2048: 512 workgroups, 58 vs 63 µs for the others; T = 512 at pos0 16384: 128
@@ -1786,9 +1887,9 @@ int launch_exact(PfCtx& c, const PrefillArgs& a) {
 template <int KV, int HW, bool QS, bool PS, bool OF32>
 int launch(PfCtx& c, const PrefillArgs& a) {
     if (c.measure) return BRASA_OK;
-    hipLaunchKernelGGL((prefill_kernel<KV, HW, QS, PS, OF32>), dim3(a.hq / HW, a.ntiles),
-                       dim3(kThreads), 0, c.stream, a);
-    return check_launch("prefill_kernel");
+    hipLaunchKernelGGL((prefill_split_kernel<KV, HW, QS, PS, OF32>), dim3(a.hq / HW, a.ntiles),
+                       dim3(2 * kThreads), 0, c.stream, a);
+    return check_launch("prefill_split_kernel");
 }
 
 // GATED: a q8_0 F16 launch on staged f16 rows (a.gate set); *gated is set when the kernel
@@ -1901,11 +2002,11 @@ int launch_prec(PfCtx& c, PrefillArgs& a, int precision) {
         // (no range flag for this stream: the exact kernel directly)
         if (precision == BRASA_PREFILL_F16) return launch_exact<KV>(c, a);
     }
-    switch (precision) {
-        case BRASA_PREFILL_F32: return launch<KV, HW, true, true, true>(c, a);
-        case BRASA_PREFILL_F16_PF32: return launch<KV, HW, false, true, false>(c, a);
-        default: return launch<KV, HW, false, false, false>(c, a);
-    }
+    if (precision == BRASA_PREFILL_F32) return launch<KV, HW, true, true, true>(c, a);
+    if constexpr (KV != BRASA_KV_F16)
+        if (precision == BRASA_PREFILL_F16_PF32) return launch<KV, HW, false, true, false>(c, a);
+    if constexpr (KV == BRASA_KV_F32) return launch<KV, HW, false, false, false>(c, a);
+    return set_error(BRASA_ERR_ARG, "flash_attention: invalid precision %d", precision);
 }
 
 template <int KV>

@@ -115,6 +115,33 @@ def test_flash_other_groups(hq, hkv):
         assert a <= 2e-3 and r <= 1e-2
 
 
+@pytest.mark.parametrize("kv,hq,hkv", [(KvType.F32, 32, 8), (KvType.F16, 16, 8),
+                                       (KvType.Q8_0, 8, 8), (KvType.Q8_0, 32, 4)])
+def test_flash_split_operand_edges(kv, hq, hkv):
+    """prefill_split_kernel (F32 precision, and F16_PF32 where the cache is not f16) at the edges
+    of its 32-key stages, its one- and two-group launches (64 keys) and its query tiles, at the
+    reference's bars. Garbage past the last key is masked."""
+    k = Kernels()
+    rng = oracle.Rng(61)
+    for tokens, pos0 in [(1, 31), (1, 32), (2, 63), (31, 1), (32, 32), (33, 64), (65, 0),
+                         (127, 2), (129, 0)]:
+        lk = pos0 + tokens
+        cap = (lk + 63) // 64 * 64
+        q = rng.vec(tokens * hq * DIM, 2.0)
+        kk, vv = rng.vec(cap * hkv * DIM, 2.0), rng.vec(cap * hkv * DIM, 3.0)
+        kk[lk * hkv * DIM:], vv[lk * hkv * DIM:] = 3e4, -3e4
+        cache = KvPair(kv, kk, vv)
+        _say(f"prefill split edges kv={kv.name_str} hq={hq} T={tokens} pos0={pos0}")
+        o32 = run_prefill(k, q, cache, tokens, hq, hkv, pos0, PrefillPrecision.F32)
+        raw, vmax = oracle.attention(q, cache.k, cache.v, tokens, hq, hkv, DIM, pos0)
+        assert oracle.worst(o32, raw, vmax) <= 1e-5, (tokens, pos0)
+        if kv == KvType.F16:
+            continue
+        op = run_prefill(k, q, cache, tokens, hq, hkv, pos0, PrefillPrecision.F16_PF32)
+        ref16, vmax = oracle.attention(q, cache.k, cache.v, tokens, hq, hkv, DIM, pos0, q16=True)
+        assert oracle.worst_f16(op, ref16, vmax) <= 1e-5, (tokens, pos0)
+
+
 def test_flash_masks_garbage_past_lk():
     # positions in [lk, cap) hold large finite garbage; results must not depend on it
     k = Kernels()
