@@ -34,7 +34,8 @@ int decode_batch_launch(const float* q, const void* const* k, const void* const*
 int prefill_launch(const float* q, const void* k, const void* v, void* o, int tokens, int hq,
                    int hkv, int pos0, int kv, int precision, bool caller_ws, void* ws,
                    size_t ws_len, hipStream_t stream, const int* layout = nullptr);
-size_t prefill_workspace_len(int tokens, int hq, int hkv, int pos0, int kv, int precision);
+size_t prefill_workspace_len(int tokens, int hq, int hkv, int pos0, int kv, int precision,
+                             size_t* required);
 void prefill_release_workspaces();
 
 namespace {
@@ -256,7 +257,7 @@ size_t brasa_flash_attention_workspace_len(brasa_attn_shape s, int precision) {
     g_err[0] = 0;
     if (prefill_check(s, precision) != BRASA_OK || s.tokens == 0) return 0;
     return prefill_workspace_len((int)s.tokens, (int)s.hq, (int)s.hkv, (int)s.pos0, s.kv,
-                                 precision);
+                                 precision, nullptr);
 }
 
 int brasa_flash_attention_ws(const float* q, const void* k, const void* v, void* o,
@@ -267,8 +268,9 @@ int brasa_flash_attention_ws(const float* q, const void* k, const void* v, void*
     if (st != BRASA_OK) return st;
     if (s.tokens == 0) return BRASA_OK;
     if (!q || !k || !v || !o) return set_error(BRASA_ERR_ARG, "flash_attention: null pointer");
-    const size_t need = prefill_workspace_len((int)s.tokens, (int)s.hq, (int)s.hkv, (int)s.pos0,
-                                              s.kv, precision);
+    // (a split that only speeds the exact precisions up is left out of a smaller workspace)
+    size_t need = 0;
+    prefill_workspace_len((int)s.tokens, (int)s.hq, (int)s.hkv, (int)s.pos0, s.kv, precision, &need);
     if (workspace_len < need || (need > 0 && !workspace))
         return set_error(BRASA_ERR_SCRATCH, "flash_attention workspace too small (%zu < %zu bytes)",
                          workspace_len, need);

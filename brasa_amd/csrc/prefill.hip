@@ -27,6 +27,7 @@
 //     phases alternate; up to two workgroups per CU), prefill_f16_kernel4 (4 waves, two per CU)
 //     and prefill_f16_kernel4s (4 waves on 32-key stages, three per CU).
 #include <atomic>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -355,13 +356,34 @@ constexpr int kStageHalves = kTile * kDim;  // one 64 x 128 f16 tile
 __device__ __forceinline__ int kswz(int r, int c) { return c ^ (r & 15); }
 __device__ __forceinline__ int vswz(int r, int c) { return c ^ (4 * (r & 3)); }
 
-constexpr int kMaxKeyParts = 8;
+constexpr int kMaxKeyParts = 32;
+constexpr int kMaxInKernelParts = 8;                // merged by the last part to arrive
 constexpr size_t kKeyPartFloats = 4 * 17 * 64 * 4;  // one part of one query tile
 
-// Key split of prefill_f16_kernel: after its two key groups have merged, each group-0 wave of
-// part `part` holds (acc, m, lsum) of its 32 queries over that part's keys. It stores them to
-// a.part (layout [query tile][part][wave][17 x 16-byte chunks][lane]: acc in 16 chunks, then
-// (m, lsum)) with device-coherent stores, waits until they are visible and counts its arrival
+// A key part's state of one wave (32 queries of one head): at 16-byte chunk c < 16 of its lane
+// the accumulator rows 4 c .. 4 c + 3, at chunk 16 (m, lsum). Layout of a.part:
+// [query tile][part][wave][17 chunks][lane].
+__device__ __forceinline__ float* part_state(const PrefillArgs& a, size_t qt, int p, int qw, int lane) {
+    return a.part + ((qt * a.kparts + p) * 4 + qw) * (17 * 64 * 4) + 4 * lane;
+}
+// Stores it for prefill_merge_kernel (the kernel boundary makes it visible). Padding columns,
+// which that kernel does not write out, are skipped.
+__device__ __forceinline__ void store_key_part(const PrefillArgs& a, int tile, int part, int qw,
+                                               int lane, const f32x16 (&acc)[4], float m, float lsum,
+                                               bool qvalid) {
+    if (!qvalid) return;
+    float* st = part_state(a, (size_t)blockIdx.x * a.ntiles + tile, part, qw, lane);
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+        *reinterpret_cast<f32x4*>(st + c * 256) =
+            f32x4{acc[c >> 2][4 * (c & 3)], acc[c >> 2][4 * (c & 3) + 1], acc[c >> 2][4 * (c & 3) + 2],
+                  acc[c >> 2][4 * (c & 3) + 3]};
+    *reinterpret_cast<f32x4*>(st + 16 * 256) = f32x4{m, lsum, 0.0f, 0.0f};
+}
+
+// Key split merged in the kernel (up to kMaxInKernelParts parts): after its two key groups have
+// merged, each group-0 wave of part `part` holds (acc, m, lsum) of its 32 queries over that
+// part's keys. It stores them to a.part (part_state) with device-coherent stores, waits until they are visible and counts its arrival
 // on the wave's counter (atomic inc wrapping at kparts - 1, so the last arrival returns it to
 // zero). The last wave to arrive loads every part's state and merges them in part order (max
 // first, then 2^(m_p - max)-weighted sums), so the result does not depend on the arrival
@@ -369,12 +391,8 @@ constexpr size_t kKeyPartFloats = 4 * 17 * 64 * 4;  // one part of one query til
 __device__ __forceinline__ bool merge_key_parts(const PrefillArgs& a, int tile, int part, int qw,
                                              int lane, f32x16 (&acc)[4], float& m_used,
                                              float& lsum) {
-    constexpr int kChunks = 17;
     const size_t qt = (size_t)blockIdx.x * a.ntiles + tile;  // query tile (head group, tile)
-    const size_t wave_floats = (size_t)kChunks * 64 * 4;
-    auto state = [&](int p) {
-        return a.part + ((qt * a.kparts + p) * 4 + qw) * wave_floats + 4 * lane;
-    };
+    auto state = [&](int p) { return part_state(a, qt, p, qw, lane); };
     float* mine = state(part);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
@@ -399,34 +417,34 @@ __device__ __forceinline__ bool merge_key_parts(const PrefillArgs& a, int tile, 
     // every slot gets a real load (parts past kparts and the own part read the own state,
     // unused): selecting between a load's result and another value before the wait would copy
     // the register before the data lands
-    f32x4 ld[kMaxKeyParts];
+    f32x4 ld[kMaxInKernelParts];
 #pragma unroll
-    for (int p = 0; p < kMaxKeyParts; ++p)
+    for (int p = 0; p < kMaxInKernelParts; ++p)
         ld[p] = ld_dev16(state(p < a.kparts && p != part ? p : part) + 16 * 256);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int p = 0; p < kMaxKeyParts; ++p) asm volatile("" : "+v"(ld[p]));
-    f32x4 ml[kMaxKeyParts];
+    for (int p = 0; p < kMaxInKernelParts; ++p) asm volatile("" : "+v"(ld[p]));
+    f32x4 ml[kMaxInKernelParts];
 #pragma unroll
-    for (int p = 0; p < kMaxKeyParts; ++p)
+    for (int p = 0; p < kMaxInKernelParts; ++p)
         ml[p] = p == part ? f32x4{m_used, lsum, 0.0f, 0.0f}
                 : p < a.kparts ? ld[p]
                                : f32x4{-INFINITY, 0.0f, 0.0f, 0.0f};
     float M = -INFINITY;
 #pragma unroll
-    for (int p = 0; p < kMaxKeyParts; ++p)
+    for (int p = 0; p < kMaxInKernelParts; ++p)
         if (p < a.kparts) M = fmaxf(M, ml[p][0]);
-    float wp[kMaxKeyParts];
+    float wp[kMaxInKernelParts];
     float L = 0.0f;
 #pragma unroll
-    for (int p = 0; p < kMaxKeyParts; ++p) {
+    for (int p = 0; p < kMaxInKernelParts; ++p) {
         wp[p] = (p >= a.kparts || ml[p][0] == -INFINITY) ? 0.0f
                                                         : __builtin_amdgcn_exp2f((ml[p][0] - M) * kLog2e);
         if (p < a.kparts) L += wp[p] * ml[p][1];
     }
     f32x16 sum[4] = {};
 #pragma unroll
-    for (int p = 0; p < kMaxKeyParts; ++p) {
+    for (int p = 0; p < kMaxInKernelParts; ++p) {
         if (p >= a.kparts) break;
         if (p == part) {
 #pragma unroll
@@ -778,7 +796,13 @@ __device__ __forceinline__ void f16_pp_tile(const PrefillArgs& a, const int tile
     PREFILL_STAMP(1 + 6 * ti + kPfMerged);
     prefetch_q();
 
-    if (a.kparts > 1 && !merge_key_parts(a, tile, part, qw, lane, acc, m_used, lsum)) return;
+    if (a.kparts > 1) {
+        if (!a.ctr) {  // merged by the next launch
+            store_key_part(a, tile, part, qw, lane, acc, m_used, lsum, qvalid);
+            return;
+        }
+        if (!merge_key_parts(a, tile, part, qw, lane, acc, m_used, lsum)) return;
+    }
     const float L = sum_xor32(lsum);
     const float inv = 1.0f / L;  // padding columns: never stored
     // this wave's 8 KB of group 0's K buffers: group 0 copies into them only after this
@@ -1239,7 +1263,13 @@ prefill_q8_kernel4(PrefillArgs a) {
 
     __syncthreads();  // every wave is done with the K stages: wave w stages its output in 8 KB of them
     if (a.taint && __builtin_amdgcn_ballot_w64(unsafe) != 0 && lane == 0) *a.taint = a.tag;
-    if (a.kparts > 1 && !merge_key_parts(a, tile, part, wave, lane, acc, m_used, lsum)) return;
+    if (a.kparts > 1) {
+        if (!a.ctr) {  // merged by the next launch
+            store_key_part(a, tile, part, wave, lane, acc, m_used, lsum, qvalid);
+            return;
+        }
+        if (!merge_key_parts(a, tile, part, wave, lane, acc, m_used, lsum)) return;
+    }
     const float L = sum_xor32(lsum);
     const float inv = 1.0f / L;
     store_o_rows(acc, inv, reinterpret_cast<uint8_t*>(&s_k[0][0]) + wave * 32 * 256, lane, a.o, tw0,
@@ -1507,7 +1537,8 @@ prefill_split_kernel(PrefillArgs a) {
     const int u = lane >> 5;         // lane half
 
     const int hg = blockIdx.x;                            // head group (fastest: spreads XCDs)
-    const int tile = a.ntiles - 1 - (int)blockIdx.y;      // heaviest query tiles first
+    const int tile = a.ntiles - 1 - (int)blockIdx.y / a.kparts;  // heaviest query tiles first
+    const int part = (int)blockIdx.y % a.kparts;          // key part of the tile
     const int h = hg * HW + (qw % HW);
     const int kh = (hg * HW) / a.group;
     const int t0 = tile * TPW;
@@ -1515,12 +1546,15 @@ prefill_split_kernel(PrefillArgs a) {
     const int lk = a.pos0 + a.tokens;
     const int kend_wg = a.pos0 + min(t0 + TPW, a.tokens);  // keys [0, kend_wg) are read
     const int kend_w = a.pos0 + min(tw0 + 32, a.tokens);   // this wave needs [0, kend_w)
-    const int nst = (kend_wg + kTileS - 1) / kTileS;       // 32-key stages
-    // launches of up to 64 keys: one group takes them all (a merge costs more than a stage)
+    const int nst_all = (kend_wg + kTileS - 1) / kTileS;   // 32-key stages of the tile
+    // this workgroup's part of them: stages [sb, sb + nst)
+    const int sb = (int)((long long)nst_all * part / a.kparts);
+    const int nst = (int)((long long)nst_all * (part + 1) / a.kparts) - sb;
+    // up to 64 keys: one group takes them all (a merge costs more than a stage)
     const int ngrp = nst <= 2 ? 1 : 2;
     if (grp >= ngrp) return;
     const int ng = (nst - grp + ngrp - 1) / ngrp;          // this group's
-    auto stage_of = [&](int i) { return ngrp * i + grp; };
+    auto stage_of = [&](int i) { return sb + ngrp * i + grp; };
 
     // ---- staging: thread (row r0, chunk ch) of the group takes rows r0 and r0 + 16 ------------
     const size_t kstride = (size_t)a.hkv * RB;
@@ -1694,8 +1728,9 @@ prefill_split_kernel(PrefillArgs a) {
     if (grp == 1) return;
     if (ngrp == 2) {
         const f32x4 ml = xch[64 * 16];
-        const float M = fmaxf(m_used, ml[0]);  // finite: group 0 saw key 0
-        const float wa = __builtin_amdgcn_exp2f((m_used - M) * kLog2e);
+        const float M = fmaxf(m_used, ml[0]);
+        // a group that saw no key of this column (a later key part's) has m = -inf, weight 0
+        const float wa = (m_used == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((m_used - M) * kLog2e);
         const float wb = (ml[0] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((ml[0] - M) * kLog2e);
         lsum = lsum * wa + ml[1] * wb;
 #pragma unroll
@@ -1705,6 +1740,11 @@ prefill_split_kernel(PrefillArgs a) {
             for (int j = 0; j < 4; ++j)
                 acc[c >> 2][4 * (c & 3) + j] = acc[c >> 2][4 * (c & 3) + j] * wa + o1[j] * wb;
         }
+        m_used = M;
+    }
+    if (a.kparts > 1) {  // merged by the next launch
+        store_key_part(a, tile, part, qw, lane, acc, m_used, lsum, qvalid);
+        return;
     }
 
     // ---- normalise and write O[t, h, d] --------------------------------------------------
@@ -1724,6 +1764,85 @@ prefill_split_kernel(PrefillArgs a) {
         // this wave's own 17 KB of the exchange area (its merge has read them): 8 KB of rows
         store_o_rows(acc, inv, reinterpret_cast<uint8_t*>(s_kv) + qw * 17 * 64 * 16, lane, a.o, tw0,
                      a.tokens, a.hq, h);
+    }
+}
+
+// The merge of a key split as a launch of its own. A split over many parts leaves more partials
+// per query tile than the one CU of the last part to arrive can load in good time (64 KB per part
+// at ~64 bytes a clock; parts waiting for each other could deadlock): here every wave loads one
+// 16-byte chunk per lane of up to 16 parts at once, so a tile's partials are spread over 16 waves
+// and all of them are in flight together. Grid (query tile x wave, 32 dims), 4 waves of one chunk
+// each. Parts are merged in part order, 16 at a time (max first, then 2^(m_p - max)-weighted
+// sums), so the result is fixed. GATED (q8_0 caches in F16 precision): when the launch that
+// converted the rows flagged a scale, the whole call is recomputed exactly from the cache.
+template <int HW, bool OF32, bool GATED>
+__global__ void __launch_bounds__(256)
+prefill_merge_kernel(PrefillArgs a) {
+    constexpr int TPW = 32 * 4 / HW;
+    constexpr int kPer = 16;
+    __shared__ __attribute__((aligned(16))) float s_o[32][36];  // [query][dim], padded rows
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    if constexpr (GATED) {
+        if (gate_open(a)) {
+            const int nwg = gridDim.x * gridDim.y;
+            for (int rw = (blockIdx.y * gridDim.x + blockIdx.x) * 4 + wave; rw < a.tokens * a.hq; rw += nwg * 4)
+                exact_row<BRASA_KV_Q8_0>(a, a.k8, a.v8, rw, lane);
+            return;
+        }
+    }
+    const int qw = blockIdx.x & 3;
+    const int qt = blockIdx.x >> 2;
+    const int hg = qt / a.ntiles, tile = qt - hg * a.ntiles;
+    const int h = hg * HW + (qw % HW);
+    const int tw0 = tile * TPW + 32 * (qw / HW);
+    const int c = 4 * blockIdx.y + wave;  // accumulator rows 4 c .. 4 c + 3
+    float M = -INFINITY, L = 0.0f;
+    f32x4 A = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p0 = 0; p0 < a.kparts; p0 += kPer) {
+        f32x4 av[kPer], ml[kPer];
+#pragma unroll
+        for (int p = 0; p < kPer; ++p) {  // (parts past the last: the last one again, unused)
+            const float* st = part_state(a, qt, min(p0 + p, a.kparts - 1), qw, lane);
+            ml[p] = *reinterpret_cast<const f32x4*>(st + 16 * 256);
+            av[p] = *reinterpret_cast<const f32x4*>(st + c * 256);
+        }
+        float Mr = -INFINITY;
+#pragma unroll
+        for (int p = 0; p < kPer; ++p)
+            if (p0 + p < a.kparts) Mr = fmaxf(Mr, ml[p][0]);
+        f32x4 Ar = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        float Lr = 0.0f;
+#pragma unroll
+        for (int p = 0; p < kPer; ++p) {
+            const bool ok = p0 + p < a.kparts && ml[p][0] != -INFINITY;
+            const float w = ok ? __builtin_amdgcn_exp2f((ml[p][0] - Mr) * kLog2e) : 0.0f;
+            Ar += w * (ok ? av[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+            Lr += w * (ok ? ml[p][1] : 0.0f);
+        }
+        const float Mn = fmaxf(M, Mr);
+        const float w0 = (M == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((M - Mn) * kLog2e);
+        const float w1 = (Mr == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((Mr - Mn) * kLog2e);
+        A = A * w0 + Ar * w1;
+        L = L * w0 + Lr * w1;
+        M = Mn;
+    }
+    const float inv = 1.0f / sum_xor32(L);
+    const int col = lane & 31, u = lane >> 5;
+    *reinterpret_cast<f32x4*>(&s_o[col][8 * wave + 4 * u]) = A * inv;
+    __syncthreads();
+    // 32 queries x 32 dims out: 8 threads per query, 4 dims each
+    const int row = threadIdx.x >> 3, d = 4 * (threadIdx.x & 7);
+    if (tw0 + row >= a.tokens) return;
+    const f32x4 y = *reinterpret_cast<const f32x4*>(&s_o[row][d]);
+    const size_t ob = ((size_t)(tw0 + row) * a.hq + h) * kDim + 32 * blockIdx.y + d;
+    if constexpr (OF32) {
+        *reinterpret_cast<f32x4*>(static_cast<float*>(a.o) + ob) = y;
+    } else {
+        uint2 w;
+        w.x = (uint32_t)f2h(as_f32(y[0])) | ((uint32_t)f2h(as_f32(y[1])) << 16);
+        w.y = (uint32_t)f2h(as_f32(y[2])) | ((uint32_t)f2h(as_f32(y[3])) << 16);
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.o) + ob) = w;
     }
 }
 
@@ -1773,6 +1892,8 @@ struct PfCtx {
     size_t used = 0;
     bool measure = false;
     size_t need = 0;
+    size_t required = 0;    // without the parts of the plan a call can do without
+    bool optional = false;  // what is taken from now on is such a part
     unsigned* ctr = nullptr;
     unsigned* taint = nullptr;
     unsigned tag = 0;
@@ -1783,10 +1904,12 @@ struct PfCtx {
     int pair = 1;
     int parts = 1;
 
+    size_t room() const { return ws ? ws_len - used : 0; }
     void* take(size_t bytes) {
         bytes = (bytes + 255) / 256 * 256;
         if (measure) {
             need += bytes;
+            if (!optional) required += bytes;
             return reinterpret_cast<void*>(static_cast<uintptr_t>(256));  // never dereferenced
         }
         if (!ws || used + bytes > ws_len) return nullptr;
@@ -1796,14 +1919,59 @@ struct PfCtx {
     }
 };
 
-// Key parts per query tile: 1 (no split) unless the launch fills at most half of the
-// workgroup slots (`slots`: CUs x workgroups per CU of the kernel) and the tiles' keys are long
-// (a short chunk after a long cached prefix, e.g. 512 tokens at pos0 16384: 128 workgroups),
-// then enough parts to fill the slots with parts of at least 16 64-key tiles each.
-int key_parts(long long wgs, int keys, int slots) {
-    int parts = 1;
-    while (parts < kMaxKeyParts && wgs * parts * 2 <= slots && keys / (64 * parts * 2) >= 16) parts *= 2;
-    return parts;
+// Key parts per query tile of a launch of `wgs` query tiles that reads `keys` keys (1: no split).
+struct KeySplit {
+    int parts;
+    bool two_step;  // merged by a launch of its own
+};
+// A split pays where the launch leaves CUs idle and a tile's keys are long. Its parts' partials
+// are 64 KB per part and tile; with few query tiles a launch of their own merges them, spread
+// over the chip, and the time left, tiles / P for the keys plus wgs * P for the partials, is
+// least at P = f sqrt(tiles / wgs), with f from each kernel's time per 64-key tile. With more
+// query tiles (and fewer parts) the last part to arrive merges them in the same launch.
+// Measured on 32 query heads over 8, f16 cache, us unsplit / in-kernel merge / own launch (best
+// parts): 8 tokens after 6000 72 / 24.1 (8 parts) / 17.7 (16); 45 after 6000 74 / 25.9 (8) /
+// 22.5 (16); 45 after 1500 24.9 / 18.0 (4) / 17.9 (6); 90 after 6000 74 / 27.2 (8) / 25.5 (10);
+// 90 after 3000 42 / 22.4 (6) / 24.1; 150 after 3000 42 / 23.5 (6) / 28.2; 400 after 3000 45 /
+// 34.9 (2) / 46.3. Short keys are left whole: 60 after 450 (8 tiles) 13.6 unsplit, 15.0 in 4
+// parts; 150 after 700 (14 tiles) 17.6, 16.6 in 3.
+KeySplit split_two_step(double f, long long wgs, int tiles, int slots, int most) {
+    const double parts = std::min(f * std::sqrt((double)tiles / wgs) + 0.5,
+                                  (double)std::min<long long>(slots / wgs, most));
+    return KeySplit{std::max((int)parts, 1), true};
+}
+KeySplit split_in_kernel(long long wgs, int tiles, int slots) {
+    const long long fit = std::min<long long>(std::min<long long>(slots / wgs, 8), tiles / 4);
+    return KeySplit{(int)std::max<long long>(fit, 1), false};
+}
+constexpr int kFewTiles = 16;  // query tiles up to which the merge is a launch of its own
+int key_tiles(int keys) { return (keys + kTile - 1) / kTile; }
+// the two-group f16 kernel, one workgroup per CU
+KeySplit key_split_f16(long long wgs, int keys) {
+    const int tiles = key_tiles(keys);
+    if (tiles < 12) return KeySplit{1, false};
+    if (wgs <= kFewTiles) return split_two_step(4.5, wgs, tiles, 256, 16);
+    const KeySplit k = split_in_kernel(wgs, tiles, 256);
+    // more than 6 parts: the own launch once the keys are long enough to pay for it
+    if (k.parts <= 6) return k;
+    return tiles >= 64 ? KeySplit{(int)(256 / wgs), true} : KeySplit{6, false};
+}
+// prefill_q8_kernel4, two workgroups per CU. The merge launch also reads the range flag, in
+// place of the launch of prefill_exact_kernel an unsplit call needs, so it pays from few tiles on
+// (8 tokens after 500: 19.1 us unsplit, 11.5 split)
+KeySplit key_split_q8(long long wgs, int keys) {
+    const int tiles = key_tiles(keys);
+    if (wgs <= kFewTiles)
+        return tiles < 4 ? KeySplit{1, false}
+                         : split_two_step(7.4, wgs, tiles, 512, std::min(tiles / 2, kMaxKeyParts));
+    return tiles < 12 ? KeySplit{1, false} : split_in_kernel(wgs, tiles, 512);
+}
+// prefill_split_kernel, one workgroup per CU (f32 cache, F32 precision: 8 tokens after 6000
+// 226 -> 26 us with 32 parts, 45 after 6000 229 -> 34 with 16, 250 after 3000 127 -> 58 with 4)
+KeySplit key_split_exact(long long wgs, int keys) {
+    const int tiles = key_tiles(keys);
+    if (tiles < (wgs <= kFewTiles ? 4 : wgs <= 64 ? 6 : 12)) return KeySplit{1, false};
+    return split_two_step(9.0, wgs, tiles, 256, std::min(tiles, kMaxKeyParts));
 }
 
 // parts within the limits of the workspace layout and the counter slot, else 1
@@ -1811,21 +1979,32 @@ int clamp_parts(int parts, long long wgs) {
     return (parts < 1 || parts > kMaxKeyParts || wgs * 4 * 16 > kPfSlotWords) ? 1 : parts;
 }
 
-// Launches `kernel` over (hq / HW) x (rows * parts) workgroups with a key split of `parts`
-// (the stream's arrival counters, the parts' partials in the call's workspace). Returns 1 when
-// the workspace or the counters are missing: the caller then launches unsplit.
-template <typename K>
-int launch_split(PfCtx& c, K kernel, const char* name, PrefillArgs b, int hw, long long wgs,
-                 int parts, int threads) {
-    void* ws = c.take((size_t)wgs * parts * kKeyPartFloats * sizeof(float));
-    if (!ws || !c.ctr) return 1;
+// Launches `kernel` over (hq / HW) x (rows * parts) workgroups with a key split of `parts` (the
+// parts' partials in the call's workspace), merged by the last part to arrive (two_step false:
+// the stream's arrival counters) or by a launch of prefill_merge_kernel. Returns 1 when the
+// workspace or the counters are missing: the caller then launches unsplit. With room for fewer
+// parts only, it splits over those.
+template <int HW, bool OF32, bool GATED, typename K>
+int launch_split(PfCtx& c, K kernel, const char* name, PrefillArgs b, long long wgs, int parts,
+                 bool two_step, int threads) {
+    const size_t unit = (size_t)wgs * kKeyPartFloats * sizeof(float);
+    if (!c.measure) {
+        if (!c.ctr) return 1;
+        parts = (int)std::min<size_t>(parts, c.room() / unit);
+        if (parts < 2) return 1;
+    }
+    void* ws = c.take(unit * parts);
     if (c.measure) return BRASA_OK;
     b.pair = 0;
     b.kparts = parts;
     b.part = static_cast<float*>(ws);
-    b.ctr = c.ctr;
-    hipLaunchKernelGGL(kernel, dim3(b.hq / hw, b.ntiles * parts), dim3(threads), 0, c.stream, b);
-    return check_launch(name);
+    b.ctr = two_step ? nullptr : c.ctr;
+    hipLaunchKernelGGL(kernel, dim3(b.hq / HW, b.ntiles * parts), dim3(threads), 0, c.stream, b);
+    const int st = check_launch(name);
+    if (st != BRASA_OK || !two_step) return st;
+    hipLaunchKernelGGL((prefill_merge_kernel<HW, OF32, GATED>), dim3((unsigned)(wgs * 4), 4), dim3(256),
+                       0, c.stream, b);
+    return check_launch("prefill_merge_kernel");
 }
 
 // q8_0 rows -> f16 rows [rows, 128], each value f16(code * scale) by the same packed f16 multiply
@@ -1886,6 +2065,15 @@ int launch_exact(PfCtx& c, const PrefillArgs& a) {
 
 template <int KV, int HW, bool QS, bool PS, bool OF32>
 int launch(PfCtx& c, const PrefillArgs& a) {
+    const long long wgs = (long long)(a.hq / HW) * a.ntiles;
+    const KeySplit ks = key_split_exact(wgs, a.pos0 + a.tokens);
+    if (ks.parts > 1) {
+        c.optional = true;
+        const int st = launch_split<HW, OF32, false>(c, prefill_split_kernel<KV, HW, QS, PS, OF32>,
+                                                     "prefill_split_kernel", a, wgs, ks.parts, true,
+                                                     2 * kThreads);
+        if (st != 1) return st;
+    }
     if (c.measure) return BRASA_OK;
     hipLaunchKernelGGL((prefill_split_kernel<KV, HW, QS, PS, OF32>), dim3(a.hq / HW, a.ntiles),
                        dim3(2 * kThreads), 0, c.stream, a);
@@ -1904,11 +2092,16 @@ int launch_f16(PfCtx& c, const PrefillArgs& a, bool* gated = nullptr) {
         PrefillArgs b = a;
         b.pair = c.pair && wgs >= 2 * 256;
         // one workgroup per CU
-        const int parts = clamp_parts(variant ? c.parts : key_parts(wgs, a.pos0 + a.tokens, 256),
-                                      wgs);
-        if (parts > 1) {
-            const int st = launch_split(c, prefill_f16_kernel<HW, PS, GATED>, "prefill_f16_kernel",
-                                        b, HW, wgs, parts, 2 * kThreads);
+        KeySplit ks = key_split_f16(wgs, a.pos0 + a.tokens);
+        if (variant) ks = KeySplit{c.parts, c.parts > kMaxInKernelParts};
+        ks.parts = clamp_parts(ks.parts, wgs);
+        if (ks.parts > 1) {
+            const int st = ks.two_step
+                ? launch_split<HW, false, GATED>(c, prefill_f16_kernel<HW, PS>, "prefill_f16_kernel",
+                                                 b, wgs, ks.parts, true, 2 * kThreads)
+                : launch_split<HW, false, GATED>(c, prefill_f16_kernel<HW, PS, GATED>,
+                                                 "prefill_f16_kernel", b, wgs, ks.parts, false,
+                                                 2 * kThreads);
             if (st != 1) return st;
         }
         if (c.measure) return BRASA_OK;
@@ -1930,14 +2123,24 @@ int launch_f16(PfCtx& c, const PrefillArgs& a, bool* gated = nullptr) {
 
 // q8_0 cache, F16 precision, small launches: prefill_q8_kernel4 (f16(code * scale) in registers)
 template <int HW>
-int launch_q8_kernel4(PfCtx& c, const PrefillArgs& a) {
+int launch_q8_kernel4(PfCtx& c, const PrefillArgs& a, bool* gated) {
     // two workgroups per CU
     const long long wgs = (long long)(a.hq / HW) * a.ntiles;
-    const int parts = clamp_parts(key_parts(wgs, a.pos0 + a.tokens, 512), wgs);
-    if (parts > 1) {
-        const int st = launch_split(c, prefill_q8_kernel4<HW>, "prefill_q8_kernel4", a, HW, wgs,
-                                    parts, kThreads);
-        if (st != 1) return st;
+    KeySplit ks = key_split_q8(wgs, a.pos0 + a.tokens);
+    ks.parts = clamp_parts(ks.parts, wgs);
+    if (ks.parts > 1) {
+        PrefillArgs b = a;
+        if (ks.two_step) {  // the merge reads the flag and recomputes the call itself
+            b.k8 = a.k;
+            b.v8 = a.v;
+            b.gate = a.taint;
+        }
+        const int st = launch_split<HW, false, true>(c, prefill_q8_kernel4<HW>, "prefill_q8_kernel4",
+                                                     b, wgs, ks.parts, ks.two_step, kThreads);
+        if (st != 1) {
+            *gated = ks.two_step;
+            return st;
+        }
     }
     if (c.measure) return BRASA_OK;
     hipLaunchKernelGGL((prefill_q8_kernel4<HW>), dim3(a.hq / HW, a.ntiles), dim3(kThreads), 0,
@@ -1954,7 +2157,7 @@ int launch_q8_via_f16(PfCtx& c, const PrefillArgs& a, bool* gated) {
     const long long rows = (long long)((a.pos0 + a.tokens + 63) / 64 * 64) * a.hkv;
     const size_t bytes = (size_t)rows * kDim * 2;
     void* ws = c.take(2 * bytes);
-    if (!ws) return launch_q8_kernel4<HW>(c, a);
+    if (!ws) return launch_q8_kernel4<HW>(c, a, gated);
     uint16_t* kd = static_cast<uint16_t*>(ws);
     uint16_t* vd = kd + rows * kDim;
     if (!c.measure) {
@@ -1982,7 +2185,9 @@ int launch_prec(PfCtx& c, PrefillArgs& a, int precision) {
         if (precision == BRASA_PREFILL_F16 && c.taint) {
             // the f16 kernels on dequantised rows when the work is large enough to hide the
             // dequantisation launch (measured: T = 384 at pos0 0 is the crossover; 128 tokens
-            // after 16384 cached positions already gain 81 -> 71 us), else the q8_0 kernel.
+            // after 16384 cached positions already gain 81 -> 71 us), else the q8_0 kernel, as
+            // for a single query tile, which reads each converted row once (30 tokens after
+            // 9000: 33.8 -> 25.9 us).
             // Both flag scales whose f16(code * scale) can leave the normal f16 range; the next
             // launch then recomputes the call exactly (the reference's F16 numerics in f32):
             // the gated two-group f16 kernel itself, or else prefill_exact_kernel, which
@@ -1990,8 +2195,8 @@ int launch_prec(PfCtx& c, PrefillArgs& a, int precision) {
             a.taint = c.taint;
             a.tag = c.tag;
             bool gated = false;
-            const int st = (long long)a.tokens * (a.pos0 + a.tokens) < 384LL * 384
-                               ? launch_q8_kernel4<HW>(c, a)
+            const int st = a.ntiles == 1 || (long long)a.tokens * (a.pos0 + a.tokens) < 384LL * 384
+                               ? launch_q8_kernel4<HW>(c, a, &gated)
                                : launch_q8_via_f16<HW>(c, a, &gated);
             if (st != BRASA_OK || gated) return st;
             PrefillArgs g = a;
@@ -2063,12 +2268,14 @@ void prefill_release_workspaces() {
 }
 
 
-size_t prefill_workspace_len(int tokens, int hq, int hkv, int pos0, int kv, int precision) {
+size_t prefill_workspace_len(int tokens, int hq, int hkv, int pos0, int kv, int precision,
+                             size_t* required) {
     PrefillArgs a = make_args(nullptr, nullptr, nullptr, nullptr, tokens, hq, hkv, pos0);
     PfCtx c;
     c.measure = true;
     c.ctr = c.taint = reinterpret_cast<unsigned*>(static_cast<uintptr_t>(256));  // never used
     run(c, a, kv, precision);
+    if (required) *required = c.required;
     return c.need;
 }
 

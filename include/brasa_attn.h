@@ -204,11 +204,13 @@ int brasa_decode_attention_batch(const float* q, const void* const* k, const voi
  * hq % hkv == 0; when hq / hkv is not in {1, 2, 4, 8} only BRASA_PREFILL_F32 is accepted
  * (BRASA_ERR_UNSUPPORTED otherwise), as the reference asserts (lib.rs:1227-1231). A launch
  * that would fill at most half of the GPU with long key ranges per query tile (a short chunk
- * after a long cached prefix, e.g. 512 tokens at pos0 16384) splits each tile's keys over up to
- * 8 workgroups; their partials go to a workspace (68 KB per part and query tile). With a q8_0
+ * after a long cached prefix, e.g. 512 tokens at pos0 16384) splits each tile's keys over several
+ * workgroups (up to 32); their partials go to a workspace (68 KB per part and query tile, at
+ * most 512 of them), merged in the same launch or, with few query tiles, by a launch of its own. With a q8_0
  * cache and BRASA_PREFILL_F16, the rows read (ceil64(pos0 + tokens) positions) are first
  * dequantised to f16 (each value f16(code * scale)) into the workspace (512 B per row of K and
- * V), and the f16 kernels run on it; small calls convert the same values in registers. When a
+ * V), and the f16 kernels run on it; small calls and calls of one query tile convert the same
+ * values in registers. When a
  * group scale lets f16(code * scale) leave the normal f16 range (|scale| >= 516, f16-subnormal,
  * inf or NaN scales) the call is recomputed exactly (the reference's F16 numerics: Q rounded
  * to f16, K / V exact, P f32) by the launch after the conversion, which reads a flag the
@@ -232,7 +234,9 @@ int brasa_flash_attention(const float* q, const void* k, const void* v, void* o,
  * No counterpart in the reference (its flash_attention encodes onto buffers the caller owns and
  * needs no scratch; lib.rs:1169-1248). Bytes of workspace brasa_flash_attention_ws needs for
  * this shape and precision: the key split's partials and the q8_0 staging the call's plan uses
- * (0 when it uses neither, or for an invalid shape).
+ * (0 when it uses neither, or for an invalid shape). BRASA_PREFILL_F32, BRASA_PREFILL_F16_PF32 on
+ * f32 and q8_0 caches and BRASA_PREFILL_F16 on f32 caches also accept less (or none), and split
+ * the keys over as many parts as fit.
  */
 size_t brasa_flash_attention_workspace_len(brasa_attn_shape shape, int precision);
 

@@ -424,7 +424,80 @@ def test_flash_calls_allocate_nothing():
     assert free1 == free0, (free0, free1)
 
 
-Q8_RANGE_CASES = [(64, 500, "k_large"), (64, 500, "v_large"), (64, 500, "tiny"),
+# (kv, precision, tokens, pos0): key splits merged by a launch of their own, with 2 to 32 parts of
+# equal and unequal lengths, one and two query tiles, and padding columns
+TWO_STEP = [(KvType.F16, "F16", 1, 767), (KvType.F16, "F16_PF32", 33, 1000),
+            (KvType.F16, "F16", 9, 7000), (KvType.F16, "F16", 80, 5000),
+            (KvType.Q8_0, "F16", 5, 300), (KvType.Q8_0, "F16", 32, 9001),
+            (KvType.Q8_0, "F16", 45, 4099), (KvType.F32, "F32", 2, 255),
+            (KvType.F32, "F32", 7, 6200), (KvType.Q8_0, "F16_PF32", 64, 700),
+            (KvType.F16, "F32", 100, 333)]
+
+
+@pytest.mark.parametrize("kv,precision,tokens,pos0", TWO_STEP)
+def test_flash_key_split_own_launch(kv, precision, tokens, pos0):
+    """Key splits merged by prefill_merge_kernel, at the bars of the unsplit kernels; repeat calls
+    give equal bits (the parts merge in a fixed order), and garbage past the last key is masked."""
+    prec = PrefillPrecision[precision]
+    synchronize()
+    assert lib().brasa_release_workspaces() == 0
+    assert Kernels.flash_attention_workspace_len(
+        AttnShape(tokens, HQ, HKV, DIM, pos0, kv), prec) > 0
+    k = Kernels()
+    rng = oracle.Rng(103 + tokens)
+    lk = pos0 + tokens
+    cap = (lk + 63) // 64 * 64
+    q = rng.vec(tokens * HQ * DIM, 2.0)
+    kk, vv = rng.vec(cap * HKV * DIM, 2.0), rng.vec(cap * HKV * DIM, 3.0)
+    kk[lk * HKV * DIM:], vv[lk * HKV * DIM:] = 3e4, -3e4
+    cache = KvPair(kv, kk, vv)
+    _say(f"prefill own-launch merge kv={kv.name_str} {precision} T={tokens} pos0={pos0}")
+    o = run_prefill(k, q, cache, tokens, HQ, HKV, pos0, prec)
+    assert np.array_equal(o, run_prefill(k, q, cache, tokens, HQ, HKV, pos0, prec))
+    if precision == "F32":
+        raw, vmax = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0)
+        assert oracle.worst(o, raw, vmax) <= 1e-5
+        return
+    ref16, vmax = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0, q16=True)
+    if precision == "F16_PF32":
+        assert oracle.worst_f16(o, ref16, vmax) <= 1e-5
+    else:
+        a, r = bars(oracle.f16_to_f32(o), ref16)
+        assert a <= 2e-3 and r <= 1e-2, (a, r)
+
+
+def test_flash_exact_split_workspace():
+    """The exact precisions' key split is optional: brasa_flash_attention_ws takes the full
+    workspace (the reference-signature call's bits), room for fewer parts, and none at all."""
+    synchronize()
+    assert lib().brasa_release_workspaces() == 0
+    k = Kernels()
+    rng = oracle.Rng(107)
+    tokens, pos0 = 40, 3000
+    cap = (pos0 + tokens + 63) // 64 * 64
+    q = rng.vec(tokens * HQ * DIM, 2.0)
+    cache = KvPair(KvType.F32, rng.vec(cap * HKV * DIM, 2.0), rng.vec(cap * HKV * DIM, 3.0))
+    shape = AttnShape(tokens, HQ, HKV, DIM, pos0, KvType.F32)
+    F32 = PrefillPrecision.F32
+    need = Kernels.flash_attention_workspace_len(shape, F32)
+    unit = 2 * HKV * 4 * 17 * 64 * 16  # one part of the launch's two query tiles a head
+    assert need >= 4 * unit
+    want = run_prefill(k, q, cache, tokens, HQ, HKV, pos0, F32)
+    raw, vmax = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0)
+    gq = DeviceBuffer.from_array(q)
+    ws = DeviceBuffer(need)
+    for size in (need, 3 * unit + 100, unit, 0):
+        ws.fill(0xFF)
+        o = DeviceBuffer(tokens * HQ * DIM * 4)
+        _say(f"prefill exact split workspace {size} of {need}")
+        k.flash_attention_ws(gq, cache.kbuf, cache.vbuf, o, shape, F32, ws if size else None, size)
+        synchronize()
+        got = o.download(np.float32).reshape(tokens, HQ, DIM)
+        assert oracle.worst(got, raw, vmax) <= 1e-5, size
+        assert size < need or np.array_equal(got, want)
+
+
+Q8_RANGE_CASES = [(9, 2500, "k_large"), (40, 4000, "k_large"), (64, 500, "k_large"), (64, 500, "v_large"), (64, 500, "tiny"),
                   (384, 0, "k_large"), (384, 0, "v_large"), (384, 0, "tiny")]
 
 
