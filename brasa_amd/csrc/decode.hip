@@ -45,13 +45,12 @@ typedef __attribute__((address_space(3))) v4s lds_v4s;
 
 constexpr int kBlock = 32;        // keys per wave iteration
 constexpr int kMinChunk = 128;    // keys per split >= DECODE_CHUNK keeps the scratch bound
-constexpr int kVStr = 144;        // V tile row stride in halves (256 B + 32 B pad)
 constexpr int kTargetWgs = 256;   // workgroups per sequence the plan aims at (one per CU)
 
 // Waves per workgroup (fixed per cache type, so results never depend on the launch).
 constexpr int kWavesF16 = 8;
 constexpr int kWavesQ8 = 8;
-constexpr int kWavesF32 = 4;
+constexpr int kWavesF32 = 8;
 // Query heads of one merge group (a workgroup's HPW head groups) the final merge's thread layout
 // covers with 8 waves (kWavesF16 / kWavesQ8).
 constexpr int kMaxMergeHeads = 16;
@@ -235,26 +234,6 @@ __device__ __forceinline__ half8 split8_sel(const float (&x)[8], bool lo_part) {
     }
     return as_half8(u32x4{w[0], w[1], w[2], w[3]});
 }
-
-// f32 caches: 8 consecutive dims of a row as MFMA operand data, split into hi and lo halves.
-struct F32Chunk {
-    f32x4 a, b;
-    __device__ __forceinline__ void load(const uint8_t* row, int d) {
-        a = ld_stream<f32x4>(row + 4 * d);
-        b = ld_stream<f32x4>(row + 4 * d + 16);
-    }
-    __device__ __forceinline__ void get(half8& hi, half8& lo) const {
-        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        split8(x, hi, lo);
-    }
-};
-
-// Per-block register state of one wave: K fragments (2 key tiles x 4 dim steps) and V chunks
-// (8 rows of 4 per lane).
-struct F32Block {
-    F32Chunk k[2][4];
-    F32Chunk v[8];
-};
 
 // A q8_0 scale s is applied as 2^e * (s * 2^-e), e = min(exponent(s), 5) (-14 for f16
 // subnormals): 2^e goes into the f16 V codes (code * 2^e, exact, made by the conversion itself,
@@ -546,189 +525,6 @@ __device__ __forceinline__ void finish_split(const DecodeArgs<NS>& a, const SeqD
     finish_split_lds<G, W, HPW>(a, sd, si, row, split, lds);
 }
 
-// ---- f32 caches (the reference's exact variant): register-staged K and V -------------------
-// Workgroup = one head group x one split, W waves walking the split's blocks w, w + W, ... K and
-// V rows are loaded into registers (the next block's loads in flight while the current block is
-// computed) and split into f16 hi + lo halves; V goes through a wave-private padded LDS tile (hi
-// and lo) to be read transposed.
-template <int G, int NS, int W>
-__global__ void __launch_bounds__(64 * W)
-decode_f32_kernel(DecodeArgs<NS> a) {
-    constexpr int RB = KvTraits<BRASA_KV_F32>::row_bytes;
-    constexpr int kVTile = 2 * kBlock * kVStr;
-
-    __shared__ __attribute__((aligned(16))) uint16_t s_v[W][kVTile];
-    __shared__ __attribute__((aligned(16))) float s_fin[finish_floats<G, W>()];
-
-    const int hg = blockIdx.x % a.ngroups;  // this workgroup's head group
-    const int col = blockIdx.x / a.ngroups;
-    const int si = seq_of(a, col);
-    const SeqDesc& sd = a.seq[si];
-    const int split = col - sd.split0;
-    const float* qseq = a.q + (size_t)si * a.hq * kDim;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int h0 = hg * G;                 // its first query head
-    const int kh = h0 / a.group;           // its KV head
-    const int c16 = lane & 15;             // MFMA row/column index
-    const int u = lane >> 4;               // MFMA k-group (8 of the 32 k-slots)
-    // The 16 MFMA columns: c < G is head h0 + c with the hi halves of the split operands,
-    // G <= c < 2 G the same head with the lo halves, the rest zero. Columns c and c ^ G add up
-    // to the f32-accurate product, so one MFMA does the work of the hi and lo passes.
-    const bool colq = c16 < G;             // this lane's column is a query head (hi half)
-    const bool col_lo = c16 >= G && c16 < 2 * G;
-    const int hcol = h0 + (c16 & (G - 1));
-
-    // ---- Q^T B-operand: k-step t holds dims 32 t + 8 u + j -----------------------------------
-    half8 qb[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        // unconditional 128-bit loads (a valid head for every lane), masked afterwards
-        const f32x4* qp = reinterpret_cast<const f32x4*>(qseq + (size_t)hcol * kDim + 32 * t + 8 * u);
-        const f32x4 q0 = qp[0], q1 = qp[1];
-        const float sc = (colq || col_lo) ? a.scale : 0.0f;
-        const float x[8] = {as_f32(q0.x * sc), as_f32(q0.y * sc), as_f32(q0.z * sc),
-                            as_f32(q0.w * sc), as_f32(q1.x * sc), as_f32(q1.y * sc),
-                            as_f32(q1.z * sc), as_f32(q1.w * sc)};  // f32, as reference
-        half8 hi, lo;
-        split8(x, hi, lo);
-        qb[t] = col_lo ? lo : hi;
-    }
-
-    // the split's 32-key blocks interleaved with the other splits' (split_blocks)
-    const SplitBlocks sb = split_blocks(sd.lk, sd.splits, split);
-    const int s0 = sb.first;
-    const int s1 = sd.lk;
-    const int nblk = sb.count;
-    const int nb = nblk > wave ? (nblk - wave + W - 1) / W : 0;  // this wave's blocks
-    const size_t kstride = (size_t)a.hkv * RB;
-    const uint8_t* kbase = sd.k + (size_t)kh * RB;
-    const uint8_t* vbase = sd.v + (size_t)kh * RB;
-    uint16_t* vt = &s_v[wave][0];
-
-    auto load = [&](F32Block& b, int jb) {
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            const uint8_t* row = kbase + (size_t)min(jb + 16 * kt + c16, s1 - 1) * kstride;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) b.k[kt][t].load(row, 32 * t + 8 * u);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            b.v[i].load(vbase + (size_t)min(jb + 4 * i + u, s1 - 1) * kstride, 8 * c16);
-    };
-
-    float m2[1] = {-INFINITY};  // running max of the column's scores, log2 domain
-    float lsum = 0.0f;          // this lane's share of the column's softmax denominator
-    f32x4 acc[8];               // O^T rows 16 dt + 4 u + i, column c16
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) acc[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    auto compute = [&](const F32Block& b, int jb) {
-        // V rows -> wave-private LDS tiles (row-major, 8 dims per lane and row; hi then lo)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            half8 hi, lo;
-            b.v[i].get(hi, lo);
-            *reinterpret_cast<half8*>(&vt[(4 * i + u) * kVStr + 8 * c16]) = hi;
-            *reinterpret_cast<half8*>(&vt[kBlock * kVStr + (4 * i + u) * kVStr + 8 * c16]) = lo;
-        }
-        // S^T tiles: rows = keys jb + 16 kt + 4 u + i, column = head
-        float x[2][4];
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            f32x4 s = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                half8 khi, klo;
-                b.k[kt][t].get(khi, klo);
-                s = mfma16(khi, qb[t], s);
-                s = mfma16(klo, qb[t], s);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[kt][i] = s[i];
-        }
-        // hi + lo columns: lanes c and c ^ G get the same sum (a + b == b + a), so both go
-        // through the softmax below with identical bits
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[kt][i] += __shfl_xor(x[kt][i], G, 64);
-        // online softmax (exp2 domain), keys past the split masked
-        float bm = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool ok = jb + 16 * kt + 4 * u + i < s1;
-                x[kt][i] = ok ? x[kt][i] * kLog2e : -INFINITY;
-                bm = fmaxf(bm, x[kt][i]);
-            }
-        bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
-        bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
-        const float mn = fmaxf(m2[0], bm);  // finite: key jb is always valid
-        const float alpha = __builtin_amdgcn_exp2f(m2[0] - mn);
-        m2[0] = mn;
-        float p[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) p[j] = __builtin_amdgcn_exp2f(x[j >> 2][j & 3] - mn);
-        float ps = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ps += p[j];
-        lsum = fmaf(lsum, alpha, ps);
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) acc[dt] *= alpha;
-
-        // O^T += V^T P^T; P^T slot j of lane (c, u) is key kappa(u, j) = j < 4 ? 4u + j : 16 + 4u + j - 4
-        // P^T B-operand: hi halves in columns < G, lo halves in [G, 2 G)
-        const half8 pb = split8_sel(p, col_lo);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        const int trc = (c16 & 3), trj = (c16 >> 2);
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-            const int col = 16 * dt + 4 * trc;
-#pragma unroll
-            for (int part = 0; part < 2; ++part) {  // V hi tile, then V lo tile
-                const uint16_t* base = vt + part * kBlock * kVStr;
-                const uint16_t* p1 = base + (4 * u + trj) * kVStr + col;
-                const uint16_t* p2 = base + (16 + 4 * u + trj) * kVStr + col;
-                const v4s lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)p1);
-                const v4s hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)p2);
-                const half8 va = __builtin_bit_cast(half8, __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
-                acc[dt] = mfma16(va, pb, acc[dt]);
-            }
-        }
-    };
-
-    // ---- stream this wave's 32-key blocks, the next block's loads in flight -----------------
-    if (nb > 0) {
-        auto blk = [&](int i) { return s0 + sb.stride * (wave + W * i); };
-        F32Block A, B;
-        load(A, blk(0));
-        // the prefetch is unconditional (rows clamp to s1 - 1): a branch around it would make
-        // the compiler wait for every outstanding load before the current block's V writes
-        int i = 0;
-        while (true) {
-            load(B, blk(i + 1));
-            compute(A, blk(i));
-            if (++i >= nb) break;
-            load(A, blk(i + 1));
-            compute(B, blk(i));
-            if (++i >= nb) break;
-        }
-    }
-
-    // ---- this wave's partial for its G heads: combine the 4 k-groups' denominators ---------
-    lsum += __shfl_xor(lsum, 16, 64);
-    lsum += __shfl_xor(lsum, 32, 64);
-    // O^T column c (hi halves of P) plus column c + G (lo halves)
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[dt][i] += __shfl_xor(acc[dt][i], G, 64);
-    finish_split<G, W, 1>(a, sd, si, hg, split, s_fin, acc, m2[0], lsum);
-}
-
 // ---- f16 caches: every load explicit --------------------------------------------------------
 // Workgroup = HPW adjacent head groups x one split of sd.chunk keys, W wave64; wave w works for
 // head group w % HPW and walks the 32-key blocks ks, ks + KS, ... of the split (ks = w / HPW,
@@ -1005,6 +801,250 @@ decode_f16_kernel(DecodeArgs<NS> a) {
     }
     DECODE_STAMP(kStampWaveDone);
     finish_split<G, W, HPW>(a, sd, si, row, split, fin, acc, mref, lsum);
+}
+
+// ---- f32 caches (the reference's exact variant) --------------------------------------------
+// K, Q, P and V stay f32 and go through v_mfma_f32_4x4x1_16b_f32 (16 blocks of 4 x 4 x 1): one
+// MFMA does 4 heads x 4 keys (or dims) in each block with no conversion, where f16 matrix
+// instructions would need every value split into hi + lo halves (the former kernel spent ~1,000
+// instructions of a 32-key block on those splits and on a transposed V tile in LDS).
+// Workgroup = one head group x one split, W wave64; a wave walks units of 16 keys (half a 32-key
+// block, so a 128-key split still feeds 8 waves), w, w + W, ... A unit is 16 loads of 16 bytes per
+// lane, K and V straight into registers, each instruction covering 4 whole rows; a wave keeps
+// two units in flight with exact waits, as decode_f16_kernel. Lane l = 16 u + c = 4 b + j.
+//  * S: block b takes dims 8 b .. 8 b + 7, A = q of head j (4 lanes: 4 heads), B = K of key
+//    4 t + j: D of lane (b, j) is the partial score of key 4 t + j for the 4 heads. The 16 blocks
+//    are summed by permlane swaps that leave tile t = u in row u, then by two DPP rotations in
+//    the row; a 4 x 4 transpose in each quad turns (key j, 4 heads) into (head j, 4 keys).
+//  * O: A = p(key, head j), B = V of that key, dims 8 c .. 8 c + 7: accumulator e of lane (u, c)
+//    holds O[4 heads][dim 8 c + e] over the keys 4 u + r, summed over u at the wave's end.
+// 8 heads per group take two sets of 4; 1 and 2 repeat the last head in the unused rows.
+// Against that kernel, 36 layers in a row: 2K keys (16.8 MB) 13.1 -> 9.5 us a layer, 129 keys 10.5
+// -> 7.6, 16K (134 MB) 30.9 -> 25.3 (4.3 -> 5.3 TB/s); its error against 64 bits is half as large.
+constexpr int kUnit = 16;  // keys
+
+// As wait_k, for the 16 loads of a ring slot.
+template <int N>
+__device__ __forceinline__ void wait_unit(u32x4 (&k)[8], u32x4 (&v)[8]) {
+    asm volatile("s_waitcnt vmcnt(%16)"
+                 : "+v"(k[0]), "+v"(k[1]), "+v"(k[2]), "+v"(k[3]), "+v"(k[4]), "+v"(k[5]),
+                   "+v"(k[6]), "+v"(k[7]), "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]),
+                   "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+                 : "n"(N)
+                 : "memory");
+}
+template <int N, int NQ>
+__device__ __forceinline__ void wait_q(u32x4 (&q)[NQ]) {
+    static_assert(NQ == 2 || NQ == 4, "one or two sets of heads");
+    if constexpr (NQ == 2)
+        asm volatile("s_waitcnt vmcnt(%2)" : "+v"(q[0]), "+v"(q[1]) : "n"(N) : "memory");
+    else
+        asm volatile("s_waitcnt vmcnt(%4)"
+                     : "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]) : "n"(N) : "memory");
+}
+// lanes 0-31: x + x of lane l ^ 32; lanes 32-63: the same of y
+__device__ __forceinline__ float swap_add32(float x, float y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// rows 0, 2: x + x of lane l ^ 16; rows 1, 3: the same of y
+__device__ __forceinline__ float swap_add16(float x, float y) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// One exchange of a 4 x 4 transpose in each quad: lanes with `hi` and their partners (CTRL: the
+// quad permutation) swap x and y across.
+template <int CTRL>
+__device__ __forceinline__ void quad_exchange(bool hi, float& x, float& y) {
+    const float got = dpp<CTRL>(hi ? x : y);
+    x = hi ? got : x;
+    y = hi ? y : got;
+}
+
+template <int G, int NS, int W>
+__global__ void __launch_bounds__(64 * W)
+decode_f32_kernel(DecodeArgs<NS> a) {
+    DECODE_STAMP(kStampStart);
+    constexpr int RB = KvTraits<BRASA_KV_F32>::row_bytes;
+    constexpr int NH = G == 8 ? 2 : 1;  // sets of 4 heads
+    __shared__ __attribute__((aligned(16))) float s_fin[finish_floats<G, W>()];
+
+    const int hg = blockIdx.x % a.ngroups;  // this workgroup's head group
+    const int col = blockIdx.x / a.ngroups;
+    const int si = seq_of(a, col);
+    const SeqDesc& sd = a.seq[si];
+    const int split = col - sd.split0;
+    const float* qseq = a.q + (size_t)si * a.hq * kDim;
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int h0 = hg * G;                 // its first query head
+    const int kh = h0 / a.group;           // its KV head
+    const int c = lane & 15, u = lane >> 4;
+    const int b = lane >> 2, j = lane & 3;
+
+    // the split's 32-key blocks interleaved with the other splits' (split_blocks), in units of 16
+    // keys; the sequence's last block may hold one unit only
+    const SplitBlocks sb = split_blocks(sd.lk, sd.splits, split);
+    const int s1 = sd.lk;
+    const int nun = 2 * sb.count - (s1 - (sb.first + sb.stride * (sb.count - 1)) <= kUnit ? 1 : 0);
+    const int nb = nun > wave ? (nun - wave + W - 1) / W : 0;  // this wave's units
+    auto key_of = [&](int i) {
+        const int x = wave + W * i;
+        return sb.first + sb.stride * (x >> 1) + kUnit * (x & 1);
+    };
+    const size_t kstride = (size_t)a.hkv * RB;
+    const uint8_t* kbase = sd.k + (size_t)kh * RB + 32 * b;
+    const uint8_t* vbase = sd.v + (size_t)kh * RB + 32 * c;
+
+    // Q: head 4 hs + j (a repeat past the group's last), dims 8 b .. 8 b + 7, loaded first
+    u32x4 qr[2 * NH];
+#pragma unroll
+    for (int hs = 0; hs < NH; ++hs) {
+        const uint8_t* qrow = reinterpret_cast<const uint8_t*>(
+            qseq + (size_t)(h0 + min(4 * hs + j, G - 1)) * kDim + 8 * b);
+        qr[2 * hs] = ld16_asm(qrow);
+        qr[2 * hs + 1] = ld16_asm(qrow + 16);
+    }
+    u32x4 kr[kRing][8], vr[kRing][8];
+    auto issue = [&](auto slot_c, int i) {
+        constexpr int S = decltype(slot_c)::value;
+        const int k0 = key_of(i);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const uint8_t* row = kbase + (size_t)min(k0 + 4 * t + j, s1 - 1) * kstride;
+            kr[S][2 * t] = ld16_asm(row);
+            kr[S][2 * t + 1] = ld16_asm(row + 16);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint8_t* row = vbase + (size_t)min(k0 + 4 * u + r, s1 - 1) * kstride;
+            vr[S][2 * r] = ld16_asm(row);
+            vr[S][2 * r + 1] = ld16_asm(row + 16);
+        }
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    if (nb > 0) issue(I0{}, 0);
+    if (nb > 1) issue(I1{}, 1);
+    // Q was issued first: it has landed when at most the units' instructions are pending
+    switch (min(nb, kRing)) {
+        case 2: wait_q<32>(qr); break;
+        case 1: wait_q<16>(qr); break;
+        default: wait_q<0>(qr); break;
+    }
+    float q[NH][8];
+    {
+        const float sc = a.scale * kLog2e;  // scores in the log2 domain
+#pragma unroll
+        for (int hs = 0; hs < NH; ++hs)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                q[hs][e] = __builtin_bit_cast(f32x4, qr[2 * hs + (e >> 2)])[e & 3] * sc;
+    }
+
+    float mref[NH], lsum[NH];  // of head 4 hs + j: reference point, this lane's denominator
+    f32x4 acc[NH][8];
+#pragma unroll
+    for (int hs = 0; hs < NH; ++hs) {
+        mref[hs] = -INFINITY;
+        lsum[hs] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[hs][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    auto step = [&](auto slot_c, int i) {
+        constexpr int S = decltype(slot_c)::value;
+        // unit i's 16 instructions were followed by those of the unit after it in the ring
+        if (i + 1 < nb) wait_unit<16>(kr[S], vr[S]);
+        else wait_unit<0>(kr[S], vr[S]);
+        if (i == 0) DECODE_STAMP(kStampFirstBlock);
+        if (i + 1 == nb) DECODE_STAMP(kStampLastBlock);
+        const int k0 = key_of(i);
+        float p[NH][4];
+#pragma unroll
+        for (int hs = 0; hs < NH; ++hs) {
+            f32x4 s[4];  // tile t: key 4 t + j, 4 heads, over dims 8 b .. 8 b + 7
+#pragma unroll
+            for (int t = 0; t < 4; ++t) s[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    s[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                        q[hs][e], __builtin_bit_cast(f32x4, kr[S][2 * t + (e >> 2)])[e & 3], s[t], 0, 0, 0);
+            float x[4];  // row u: key 4 u + j of heads 0..3, then of head j the keys 4 u + r
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const float y = swap_add16(swap_add32(s[0][h], s[2][h]), swap_add32(s[1][h], s[3][h]));
+                x[h] = y + dpp<0x128>(y);     // row_ror:8
+                x[h] = x[h] + dpp<0x124>(x[h]);  // row_ror:4
+            }
+            quad_exchange<0xB1>(j & 1, x[0], x[1]);
+            quad_exchange<0xB1>(j & 1, x[2], x[3]);
+            quad_exchange<0x4E>(j & 2, x[0], x[2]);
+            quad_exchange<0x4E>(j & 2, x[1], x[3]);
+            if (k0 + kUnit > s1) {  // the sequence's last unit: keys past its end get -inf
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (k0 + 4 * u + r >= s1) x[r] = -INFINITY;
+            }
+            const float bm = max_rows(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));  // finite
+            // lazy reference point: rescale O only when some head's max grew by more than 2^8
+            if (__builtin_amdgcn_ballot_w64(bm > mref[hs] + kLazyRescale) != 0) {
+                const float mn = fmaxf(mref[hs], bm);
+                const float alpha = __builtin_amdgcn_exp2f(mref[hs] - mn);  // of head j
+                mref[hs] = mn;
+                lsum[hs] *= alpha;
+                // component h of every accumulator belongs to head h: the factor of lane h of
+                // the quad
+                const f32x4 ah = f32x4{dpp<0x00>(alpha), dpp<0x55>(alpha), dpp<0xaa>(alpha),
+                                       dpp<0xff>(alpha)};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[hs][e] *= ah;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                p[hs][r] = __builtin_amdgcn_exp2f(x[r] - mref[hs]);
+                lsum[hs] += p[hs][r];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int hs = 0; hs < NH; ++hs)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    acc[hs][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                        p[hs][r], __builtin_bit_cast(f32x4, vr[S][2 * r + (e >> 2)])[e & 3], acc[hs][e],
+                        0, 0, 0);
+        if (i + kRing < nb) issue(slot_c, i + kRing);
+    };
+    for (int i0 = 0; i0 < nb; i0 += kRing) {
+        step(I0{}, i0);
+        if (i0 + 1 >= nb) break;
+        step(I1{}, i0 + 1);
+    }
+
+    // ---- the split's end: sum the key quarters u, lane (u, c) keeps heads u and 4 + u --------
+    DECODE_STAMP(kStampWaveDone);
+#pragma unroll
+    for (int hs = 0; hs < NH; ++hs) {
+        const float l = sum_rows(lsum[hs]);
+        float o8[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            o8[e] = swap_add16(swap_add32(acc[hs][e][0], acc[hs][e][2]),
+                               swap_add32(acc[hs][e][1], acc[hs][e][3]));
+        if (4 * hs + u < G) {
+            float* dst = s_fin + (wave * G + 4 * hs + u) * kDim + 8 * c;  // m_acc [W][G][128]
+            *reinterpret_cast<f32x4*>(dst) = f32x4{o8[0], o8[1], o8[2], o8[3]};
+            *reinterpret_cast<f32x4*>(dst + 4) = f32x4{o8[4], o8[5], o8[6], o8[7]};
+        }
+        if (lane < 4 && 4 * hs + j < G)  // m_ml [W][G][2]
+            *reinterpret_cast<f32x2*>(s_fin + W * G * kDim + (wave * G + 4 * hs + j) * 2) =
+                f32x2{mref[hs], l};
+    }
+    finish_split_lds<G, W, 1>(a, sd, si, hg, split, s_fin);
 }
 
 // ---- q8_0 caches: the f16 kernel's structure with codes and scales staged in LDS -----------
