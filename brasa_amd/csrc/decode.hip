@@ -55,12 +55,13 @@ constexpr int kWavesF32 = 8;
 // covers with 8 waves (kWavesF16 / kWavesQ8).
 constexpr int kMaxMergeHeads = 16;
 // Merge size bounds of the plan, in (query heads x splits) of a merge group; the last workgroup
-// loads 520 bytes per (query head, split). Up to kMergeWorkSmall (66 KB) for any layout; up to
+// loads 520 bytes per (query head, split). Up to kMergeWorkSmall (106 KB) for any layout; up to
 // kMergeWorkLong (~200 KB) when splits are long (>= kLongChunk keys), where streaming several KV
 // heads per workgroup gains more than the larger merge costs.
-constexpr int kMergeWorkSmall = 128;
+constexpr int kMergeWorkSmall = 208;
 constexpr int kMergeWorkLong = 384;
 constexpr int kLongChunk = 512;
+constexpr int kLongSplit = 1024;  // keys per split above which a large batch takes more rounds
 
 // Sequences per launch: their descriptors travel in the kernel arguments (no device-side
 // metadata, so a call allocates and copies nothing).
@@ -157,18 +158,19 @@ __device__ __forceinline__ int seq_of(const DecodeArgs<NS>& a, int col) {
 // fastest, the heads of one split sat on eight different XCDs and every shared line was
 // fetched from HBM twice. Here the workgroups b, b + 8, ... (one XCD) take the rows of a
 // column one after another, so the heads of a split share their lines in one L2 (16K keys:
-// 21.5 -> 19.4 us). Any bijection is correct; this one needs the column count to be a
-// multiple of 8 and falls back to rows-fastest otherwise.
+// 21.5 -> 19.4 us). Any bijection is correct; the columns past the last multiple of 8 (batches,
+// and lengths such as 4097: 26 splits, 10.7 -> 10.3 us) go rows-fastest.
 __device__ __forceinline__ void xcd_grid_pos(int rows, int& row, int& col) {
     const int b = blockIdx.x;
-    const int cols = gridDim.x / rows;
-    if (cols % 8 == 0) {
+    const int cols8 = (gridDim.x / rows) & ~7;
+    if (b < cols8 * rows) {
         const int j = b >> 3;
         row = j % rows;
         col = (j / rows) * 8 + (b & 7);
     } else {
-        row = b % rows;
-        col = b / rows;
+        const int r = b - cols8 * rows;
+        row = r % rows;
+        col = cols8 + r / rows;
     }
 }
 
@@ -861,24 +863,30 @@ __device__ __forceinline__ void quad_exchange(bool hi, float& x, float& y) {
     y = hi ? y : got;
 }
 
-template <int G, int NS, int W>
+template <int G, int NS, int HPW, int W>
 __global__ void __launch_bounds__(64 * W)
 decode_f32_kernel(DecodeArgs<NS> a) {
     DECODE_STAMP(kStampStart);
     constexpr int RB = KvTraits<BRASA_KV_F32>::row_bytes;
     constexpr int NH = G == 8 ? 2 : 1;  // sets of 4 heads
+    constexpr int KS = W / HPW;
     __shared__ __attribute__((aligned(16))) float s_fin[finish_floats<G, W>()];
 
-    const int hg = blockIdx.x % a.ngroups;  // this workgroup's head group
-    const int col = blockIdx.x / a.ngroups;
+    // grid: (split column, row of HPW head groups), rows innermost
+    const int rows = (a.ngroups + HPW - 1) / HPW;
+    const int row = blockIdx.x % rows;
+    const int col = blockIdx.x / rows;
     const int si = seq_of(a, col);
     const SeqDesc& sd = a.seq[si];
     const int split = col - sd.split0;
     const float* qseq = a.q + (size_t)si * a.hq * kDim;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int h0 = hg * G;                 // its first query head
-    const int kh = h0 / a.group;           // its KV head
+    const int ks = wave / HPW;
+    const int hg = row * HPW + wave % HPW;       // this wave's head group
+    const bool hg_ok = hg < a.ngroups;
+    const int h0 = min(hg, a.ngroups - 1) * G;   // its first query head
+    const int kh = h0 / a.group;                 // its KV head
     const int c = lane & 15, u = lane >> 4;
     const int b = lane >> 2, j = lane & 3;
 
@@ -887,9 +895,10 @@ decode_f32_kernel(DecodeArgs<NS> a) {
     const SplitBlocks sb = split_blocks(sd.lk, sd.splits, split);
     const int s1 = sd.lk;
     const int nun = 2 * sb.count - (s1 - (sb.first + sb.stride * (sb.count - 1)) <= kUnit ? 1 : 0);
-    const int nb = nun > wave ? (nun - wave + W - 1) / W : 0;  // this wave's units
+    // this wave's units: ks, ks + KS, ...
+    const int nb = (hg_ok && nun > ks) ? (nun - ks + KS - 1) / KS : 0;
     auto key_of = [&](int i) {
-        const int x = wave + W * i;
+        const int x = ks + KS * i;
         return sb.first + sb.stride * (x >> 1) + kUnit * (x & 1);
     };
     const size_t kstride = (size_t)a.hkv * RB;
@@ -911,15 +920,15 @@ decode_f32_kernel(DecodeArgs<NS> a) {
         const int k0 = key_of(i);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint8_t* row = kbase + (size_t)min(k0 + 4 * t + j, s1 - 1) * kstride;
-            kr[S][2 * t] = ld16_asm(row);
-            kr[S][2 * t + 1] = ld16_asm(row + 16);
+            const uint8_t* krow = kbase + (size_t)min(k0 + 4 * t + j, s1 - 1) * kstride;
+            kr[S][2 * t] = ld16_asm(krow);
+            kr[S][2 * t + 1] = ld16_asm(krow + 16);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const uint8_t* row = vbase + (size_t)min(k0 + 4 * u + r, s1 - 1) * kstride;
-            vr[S][2 * r] = ld16_asm(row);
-            vr[S][2 * r + 1] = ld16_asm(row + 16);
+            const uint8_t* vrow = vbase + (size_t)min(k0 + 4 * u + r, s1 - 1) * kstride;
+            vr[S][2 * r] = ld16_asm(vrow);
+            vr[S][2 * r + 1] = ld16_asm(vrow + 16);
         }
     };
     using I0 = std::integral_constant<int, 0>;
@@ -1044,7 +1053,7 @@ decode_f32_kernel(DecodeArgs<NS> a) {
             *reinterpret_cast<f32x2*>(s_fin + W * G * kDim + (wave * G + 4 * hs + j) * 2) =
                 f32x2{mref[hs], l};
     }
-    finish_split_lds<G, W, 1>(a, sd, si, hg, split, s_fin);
+    finish_split_lds<G, W, HPW>(a, sd, si, row, split, s_fin);
 }
 
 // ---- q8_0 caches: the f16 kernel's structure with codes and scales staged in LDS -----------
@@ -1693,35 +1702,29 @@ int launch_hpw(const DecodeArgs<NS>& a, int cols, hipStream_t stream) {
     constexpr int W = KernelFor<KV>::W;
     const int rows = (a.ngroups + HPW - 1) / HPW;
     const dim3 grid(cols * rows), block(64 * W);
-    if constexpr (KV == BRASA_KV_F16) {
+    if constexpr (KV == BRASA_KV_F32) {
+        hipLaunchKernelGGL((decode_f32_kernel<G, NS, HPW, W>), grid, block, 0, stream, a);
+        return check_launch("decode_f32_kernel");
+    } else if constexpr (KV == BRASA_KV_F16) {
         hipLaunchKernelGGL((decode_f16_kernel<G, NS, HPW, W>), grid, block, 0, stream, a);
         return check_launch("decode_f16_kernel");
+    } else if constexpr (G == 4) {
+        hipLaunchKernelGGL((decode_q8h_kernel<NS, HPW, W>), grid, block, 0, stream, a);
+        return check_launch("decode_q8h_kernel");
     } else {
-        if constexpr (G == 4) {
-            hipLaunchKernelGGL((decode_q8h_kernel<NS, HPW, W>), grid, block, 0, stream, a);
-            return check_launch("decode_q8h_kernel");
-        } else {
-            hipLaunchKernelGGL((decode_q8_kernel<G, NS, HPW, W>), grid, block, 0, stream, a);
-            return check_launch("decode_q8_kernel");
-        }
+        hipLaunchKernelGGL((decode_q8_kernel<G, NS, HPW, W>), grid, block, 0, stream, a);
+        return check_launch("decode_q8_kernel");
     }
 }
 
 template <int KV, int G, int NS>
 int launch(const DecodeArgs<NS>& a, int hpw, int cols, hipStream_t stream) {
-    if constexpr (KV == BRASA_KV_F32) {
-        constexpr int W = KernelFor<KV>::W;
-        hipLaunchKernelGGL((decode_f32_kernel<G, NS, W>), dim3(cols * a.ngroups), dim3(64 * W), 0,
-                           stream, a);
-        return check_launch("decode_f32_kernel");
-    } else {
-        if (hpw == 1) return launch_hpw<KV, G, NS, 1>(a, cols, stream);
-        if constexpr (2 * G <= kMaxMergeHeads)
-            if (hpw == 2) return launch_hpw<KV, G, NS, 2>(a, cols, stream);
-        if constexpr (4 * G <= kMaxMergeHeads)
-            if (hpw == 4) return launch_hpw<KV, G, NS, 4>(a, cols, stream);
-        return set_error(BRASA_ERR_UNSUPPORTED, "decode: %d head groups per workgroup not compiled", hpw);
-    }
+    if (hpw == 1) return launch_hpw<KV, G, NS, 1>(a, cols, stream);
+    if constexpr (2 * G <= kMaxMergeHeads)
+        if (hpw == 2) return launch_hpw<KV, G, NS, 2>(a, cols, stream);
+    if constexpr (4 * G <= kMaxMergeHeads)
+        if (hpw == 4) return launch_hpw<KV, G, NS, 4>(a, cols, stream);
+    return set_error(BRASA_ERR_UNSUPPORTED, "decode: %d head groups per workgroup not compiled", hpw);
 }
 
 template <int KV, int NS>
@@ -1784,38 +1787,69 @@ int arrival_counters(hipStream_t stream, unsigned** out) {
 
 }  // namespace
 
-// Split length for `keys` keys spread over about kTargetWgs / ngroups splits: a multiple of 32
-// keys and at least 128 keys, so a sequence of lk keys has at most ceil(lk / 128) splits and its
-// partials fit the reference's decode_partials_len(hq, lk).
-static long long split_chunk(long long keys, int ngroups) {
-    const int target = ngroups >= kTargetWgs ? 1 : kTargetWgs / ngroups;
-    long long chunk = (keys + target - 1) / target;
-    chunk = (chunk + kBlock - 1) / kBlock * kBlock;
-    return chunk < kMinChunk ? kMinChunk : chunk;
+// The shortest split length with which n sequences of lengths lk (`total` keys) make at most
+// `most` splits: a multiple of 32 keys and at least 128 keys, so a sequence of lk keys has at most
+// ceil(lk / 128) splits and its partials fit the reference's decode_partials_len(hq, lk). With
+// fewer splits allowed than sequences, one split each.
+static int split_chunk(const int* lk, int n, long long total, int lk_max, int most) {
+    auto blocks = [](long long keys) {
+        return std::max((unsigned)((keys + kBlock - 1) / kBlock), (unsigned)(kMinChunk / kBlock));
+    };
+    unsigned lo = blocks((total + most - 1) / most), hi = blocks(lk_max);  // in 32-key blocks
+    if (n == 1) return (int)lo * kBlock;
+    // a sequence adds at most one split to its share of total / chunk
+    if (most > n) hi = std::min(hi, blocks((total + most - n - 1) / (most - n)));
+    while (lo < hi) {
+        const unsigned mid = (lo + hi) / 2, chunk = mid * kBlock;
+        unsigned splits = 0;
+        for (int i = 0; i < n; ++i) splits += ((unsigned)lk[i] + chunk - 1) / chunk;
+        if (splits <= (unsigned)most) hi = mid;
+        else lo = mid + 1;
+    }
+    return (int)lo * kBlock;
 }
 
 // Launch plan: head groups per workgroup (HPW) and one split length for every sequence of the
-// launch. Workgroups that read several adjacent KV heads load the HBM channels evenly (with one
-// KV head per workgroup, the heads whose rows sit on the slower channels arrive ~2 us late at
-// 16K keys), but each merge group then has HPW * G query heads; the plan takes the largest HPW
-// whose merge (query heads x splits of the longest sequence) stays within the bounds above,
-// with the split length set for ~kTargetWgs workgroups. f32 caches use one head group per workgroup.
-// A function of the lengths and head counts only, so a call's result never depends on anything
-// else.
+// launch. A function of the lengths and head counts only, so a call's result never depends on
+// anything else.
+//  * Split length: the shortest that keeps the launch within one workgroup per CU (a workgroup
+//    fills its CU, so one workgroup more would run after the others: a batch of 8 sequences of
+//    1024 to 16384 keys, 75K in all, took 72 us with 276 workgroups and takes 50 with 256). Where
+//    that leaves a batch of many sequences and heads (fewer than four splits each) with splits of
+//    more than kLongSplit keys, it takes two or four rounds of shorter ones instead, which balance
+//    better (32 KV heads, the same batch: 177 against 187 us; 8 KV heads: 53 against 50).
+//  * HPW: workgroups that read several adjacent KV heads load the HBM channels evenly (with one
+//    KV head per workgroup, the heads whose rows sit on the slower channels arrive ~2 us late at
+//    16K keys), but each merge group then has HPW * G query heads. The plan takes the largest HPW
+//    whose merge (query heads x splits of the longest sequence) stays within the bounds above,
+//    and which still has a workgroup for most of the CUs: below that it only makes the waves'
+//    work longer (f16, 32 heads over 8: 257 keys 10.4 us with 4, 8.6 with 2, 7.2 with 1; 1000
+//    keys 12.2 / 9.5 / 7.8; 2000 keys 9.6 with 2, 7.9 with 1). f32 rows are 512 bytes, and two
+//    heads per workgroup do as well as four (32 KV heads, 16K: 90 us, 97 with four).
 DecodePlan decode_plan(const int* lk, int n, int ngroups, int G, int kv) {
-    long long total = 0, lk_max = 0;
+    long long total = 0;
+    int lk_max = 0;
     for (int i = 0; i < n; ++i) {
         total += lk[i];
-        lk_max = std::max<long long>(lk_max, lk[i]);
+        lk_max = std::max(lk_max, lk[i]);
     }
-    for (int hpw = 4; hpw >= 1; hpw >>= 1) {
-        if (hpw > 1 && (kv == BRASA_KV_F32 || hpw * G > kMaxMergeHeads || hpw > ngroups)) continue;
+    for (int hpw = kv == BRASA_KV_F32 ? 2 : 4; hpw >= 1; hpw >>= 1) {
+        if (hpw > 1 && (hpw * G > kMaxMergeHeads || hpw > ngroups)) continue;
         const int rows = (ngroups + hpw - 1) / hpw;
-        const long long chunk = split_chunk(total, rows);
-        const long long splits = (lk_max + chunk - 1) / chunk;
-        const long long work = splits * hpw * G;
-        if (hpw == 1 || work <= kMergeWorkSmall || (chunk >= kLongChunk && work <= kMergeWorkLong))
-            return DecodePlan{(int)chunk, (int)splits, hpw};
+        int chunk = 0;
+        for (int wgs = kTargetWgs; wgs <= 4 * kTargetWgs; wgs *= 2) {
+            chunk = split_chunk(lk, n, total, lk_max, std::max(wgs / rows, 1));
+            if (chunk <= kLongSplit || n * rows < kTargetWgs / 4) break;
+        }
+        const int splits = (int)(((long long)lk_max + chunk - 1) / chunk);
+        if (hpw > 1) {
+            const long long work = (long long)splits * hpw * G;
+            if (work > kMergeWorkSmall && !(chunk >= kLongChunk && work <= kMergeWorkLong)) continue;
+            long long wgs = 0;
+            for (int i = 0; i < n; ++i) wgs += ((unsigned)lk[i] + chunk - 1) / chunk;
+            if (wgs * rows < kTargetWgs * 3 / 4) continue;
+        }
+        return DecodePlan{chunk, splits, hpw};
     }
     return DecodePlan{kMinChunk, 1, 1};  // not reached
 }

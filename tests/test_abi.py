@@ -311,6 +311,32 @@ def _blocks(lk, splits, split):
     return [f.value + st.value * i for i in range(n.value)]
 
 
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (32, 4), (16, 8), (32, 32), (20, 5)])
+@pytest.mark.parametrize("kv", [KvType.F16, KvType.Q8_0, KvType.F32])
+def test_decode_plan_fills_the_gpu_once(hq, hkv, kv):
+    """One workgroup fills a CU, so a launch of up to 256 runs in one round: the plan cuts the
+    shortest splits that keep within it (32 keys shorter would not, unless 128 keys are reached),
+    or, for many sequences and heads with long splits, within 512 or 1024. Several head groups
+    share a workgroup only where at least 192 workgroups are left."""
+    import random
+    r = random.Random(hq * 100 + hkv)
+    for _ in range(200):
+        n = r.choice([1, 1, 2, 5, 8, 16, 40, 64])
+        lens = [int(2 ** r.uniform(0, 14.5)) for _ in range(n)]
+        chunk, hpw, splits = _plan(lens, hq, hkv, kv)
+        rows = -(-hkv // hpw)
+        wgs = lambda c: rows * sum(-(-lk // c) for lk in lens)
+        assert wgs(chunk) == rows * sum(splits)
+        if hpw > 1:
+            assert wgs(chunk) >= 192 and (kv != KvType.F32 or hpw == 2)
+        least = next((w for w in (256, 512, 1024) if wgs(chunk) <= w), None)
+        if least is None:  # more sequences and heads than that
+            assert n * rows > 256
+        elif chunk > 128 and n * rows <= least:
+            assert wgs(chunk - 32) > least
+        assert least == 256 or n * rows >= 64
+
+
 @pytest.mark.parametrize("lens,hq,hkv,kv", [
     ([1], 32, 8, KvType.F16), ([37], 32, 8, KvType.Q8_0), ([128], 32, 8, KvType.F16),
     ([129], 32, 8, KvType.F16), ([2048], 32, 8, KvType.F16), ([4096], 32, 8, KvType.Q8_0),

@@ -72,6 +72,23 @@ def test_batch_other_groups(group):
         assert oracle.worst(got[i], want, vmax) <= 1e-5
 
 
+@pytest.mark.parametrize("kv,group", [(KvType.F32, 4), (KvType.F32, 8), (KvType.F16, 4),
+                                      (KvType.F16, 8), (KvType.Q8_0, 4), (KvType.Q8_0, 2)])
+def test_batch_several_heads_per_workgroup(kv, group):
+    """Five KV heads, two or four to a workgroup: the last grid row holds one head group and
+    places past it. Lengths around the edges of units, blocks and splits."""
+    from test_abi import _plan
+    hkv = 5
+    hq = hkv * group
+    lens = [1500, 1, 900, 33, 1201, 16, 700, 1024, 129, 1100, 17, 1333, 800, 511, 1250, 950, 640]
+    assert _plan(lens, hq, hkv, kv)[1] > 1
+    k = Kernels()
+    qs, caches, got = run_batch(k, kv, lens, 53, hq=hq, hkv=hkv)
+    for i, lk in enumerate(lens):
+        want, vmax = oracle.attention(qs[i], caches[i].k, caches[i].v, 1, hq, hkv, DIM, lk - 1)
+        assert oracle.worst(got[i], want, vmax) <= 1e-5, (i, lk)
+
+
 @pytest.mark.parametrize("kv", [KvType.F16, KvType.Q8_0])
 def test_ragged_batch_rescale_after_first_block(kv):
     """The ragged batch (four adjacent KV heads per workgroup) on inputs whose scores jump
