@@ -8,15 +8,15 @@
 // into the cache from pos0 on in the cache type (store_kv rounding: f16 RNE or q8_0).
 //
 // Design: lane l of a wave64 holds elements l and l + 64 of a 128-element row (exactly a RoPE
-// pair); each wave takes four consecutive rows and issues every load of the four (row, norm
-// weights, cos/sin) before the first reduction, so a wave keeps 4 rows of reads in flight (in-place
-// writes of one row could otherwise alias the next row's loads and serialise them). The sum of
-// squares has one fixed order shared with the unfused rms_norm kernel (lane partials in index
-// order, then a butterfly inside 16-lane rows by DPP and across rows by v_permlane16/32_swap), so
-// fused and unfused results are identical bits, as the reference's fused test demands
-// (crates/kernels/tests/fused.rs:8-98). The q8_0 groups of 32 are half-waves: the group amax is
-// the same exchanges without the last one. HBM-bound: T * (hq + 2 hkv) * 512 B read, q/k
-// rewritten, cache rows written.
+// pair); each wave takes four consecutive rows (one in small launches) and issues every load of
+// the four (row, norm weights, cos/sin) before the first reduction, so a wave keeps 4 rows of
+// reads in flight (in-place writes of one row could otherwise alias the next row's loads and
+// serialise them). The sum of squares has one fixed order shared with the unfused rms_norm kernel
+// (lane partials in index order, then a butterfly inside 16-lane rows by DPP and across rows by
+// v_permlane16/32_swap), so fused and unfused results are identical bits, as the reference's
+// fused test demands (crates/kernels/tests/fused.rs:8-98). The q8_0 groups of 32 are half-waves:
+// the group amax is the same exchanges without the last one. HBM-bound: T * (hq + 2 hkv) * 512 B
+// read, q/k rewritten, cache rows written.
 #include <cmath>
 #include <vector>
 
@@ -27,7 +27,7 @@ namespace {
 
 constexpr int kRowsPerWg = 4;    // rms_norm: one row per wave
 constexpr int kWavesPerWg = 4;   // qk_norm_rope_store
-constexpr int kRowsPerWave = 4;
+constexpr int kRowsPerWave = 4;  // of launches that fill the GPU (launch_qkv)
 
 // Sum over the wave of the per-lane partials in one fixed order: the 16-lane DPP butterfly, then
 // lanes l ^ 16 and l ^ 32. Partners always add the same two values, so every lane ends with
@@ -135,22 +135,22 @@ struct QkvArgs {
 // Row gr of T * (hq + 2 hkv): within a token, first the hq query heads, then the hkv key heads,
 // then the hkv value heads (the reference's order, qkv.metal:59-61). Wave w takes rows
 // 4 w .. 4 w + 3.
-template <int KV>
+template <int KV, int RPW>
 __global__ void __launch_bounds__(64 * kWavesPerWg) qk_norm_rope_store_kernel(QkvArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t s_stage[kWavesPerWg][KV == BRASA_KV_Q8_0 ? kQ8Row : 4];
-    const int gr0 = (blockIdx.x * kWavesPerWg + (threadIdx.x >> 6)) * kRowsPerWave;
+    const int gr0 = (blockIdx.x * kWavesPerWg + (threadIdx.x >> 6)) * RPW;
     const int lane = threadIdx.x & 63;
     uint8_t* stage = s_stage[threadIdx.x >> 6];
     if (gr0 >= a.rows) return;
     const int per_tok = a.hq + 2 * a.hkv;
-    float x0[kRowsPerWave], x1[kRowsPerWave], w0[kRowsPerWave], w1[kRowsPerWave];
-    float c[kRowsPerWave], sn[kRowsPerWave];
-    float* dst[kRowsPerWave];
-    size_t crow[kRowsPerWave];
-    int kind[kRowsPerWave];  // 0 q, 1 k, 2 v, 3 past the last row
+    float x0[RPW], x1[RPW], w0[RPW], w1[RPW];
+    float c[RPW], sn[RPW];
+    float* dst[RPW];
+    size_t crow[RPW];
+    int kind[RPW];  // 0 q, 1 k, 2 v, 3 past the last row
     // every load of the four rows first
 #pragma unroll
-    for (int j = 0; j < kRowsPerWave; ++j) {
+    for (int j = 0; j < RPW; ++j) {
         const int gr = gr0 + j;
         kind[j] = 3;
         if (gr >= a.rows) continue;
@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(64 * kWavesPerWg) qk_norm_rope_store_kernel(Qk
         sn[j] = a.sin_t[tp];
     }
 #pragma unroll
-    for (int j = 0; j < kRowsPerWave; ++j) {
+    for (int j = 0; j < RPW; ++j) {
         if (kind[j] == 3) break;
         if (kind[j] == 2) {
             store_row<KV>(a.vc, crow[j], lane, x0[j], x1[j], stage);
@@ -195,6 +195,24 @@ __global__ void __launch_bounds__(64 * kWavesPerWg) qk_norm_rope_store_kernel(Qk
         dst[j][lane + 64] = y1;
         if (kind[j] == 1) store_row<KV>(a.kc, crow[j], lane, y0, y1, stage);
     }
+}
+
+template <int KV, int RPW>
+void launch_rows(const QkvArgs& a, hipStream_t stream) {
+    const int per_wg = kWavesPerWg * RPW;
+    hipLaunchKernelGGL((qk_norm_rope_store_kernel<KV, RPW>), dim3((unsigned)((a.rows + per_wg - 1) / per_wg)),
+                       dim3(64 * kWavesPerWg), 0, stream, a);
+}
+// One row per wave while every row can have a wave of its own at once (256 CUs x 32 waves): a
+// wave's rows are a serial chain of reductions, square roots and divides, and the decode step's
+// one token is 48 rows (a step's launch pair, store and decode, at 4K: 13.3 -> 11.9 us a layer,
+// q8_0 15.9 -> 13.8). Above that four rows, whose loads travel together (T = 2048: 20.6 us, 21.0
+// with one).
+constexpr int kOneRowEach = 256 * 32;
+template <int KV>
+void launch_qkv(const QkvArgs& a, hipStream_t stream) {
+    if (a.rows <= kOneRowEach) launch_rows<KV, 1>(a, stream);
+    else launch_rows<KV, kRowsPerWave>(a, stream);
 }
 
 unsigned row_blocks(size_t rows) { return (unsigned)((rows + kRowsPerWg - 1) / kRowsPerWg); }
@@ -238,18 +256,10 @@ int qk_norm_rope_store_launch(int kv, float* q, float* k, const float* v, const 
     a.rows = (int)(tokens * (hq + 2 * hkv));
     a.eps = eps;
     if (a.rows == 0) return BRASA_OK;
-    const int per_wg = kWavesPerWg * kRowsPerWave;
-    const dim3 grid((unsigned)((a.rows + per_wg - 1) / per_wg)), block(64 * kWavesPerWg);
     switch (kv) {
-        case BRASA_KV_F32:
-            hipLaunchKernelGGL(qk_norm_rope_store_kernel<BRASA_KV_F32>, grid, block, 0, stream, a);
-            break;
-        case BRASA_KV_F16:
-            hipLaunchKernelGGL(qk_norm_rope_store_kernel<BRASA_KV_F16>, grid, block, 0, stream, a);
-            break;
-        case BRASA_KV_Q8_0:
-            hipLaunchKernelGGL(qk_norm_rope_store_kernel<BRASA_KV_Q8_0>, grid, block, 0, stream, a);
-            break;
+        case BRASA_KV_F32: launch_qkv<BRASA_KV_F32>(a, stream); break;
+        case BRASA_KV_F16: launch_qkv<BRASA_KV_F16>(a, stream); break;
+        case BRASA_KV_Q8_0: launch_qkv<BRASA_KV_Q8_0>(a, stream); break;
         default:
             return set_error(BRASA_ERR_ARG, "qk_norm_rope_store: invalid kv type %d", kv);
     }

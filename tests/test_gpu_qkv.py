@@ -168,3 +168,32 @@ def test_qk_norm_rope_store_writes_at_pos0_view():
     assert np.all(kk[:lo] == 0x33) and np.all(kk[hi:] == 0x33)
     assert np.all(vv[:lo] == 0x44) and np.all(vv[hi:] == 0x44)
     assert np.array_equal(kk[lo:hi], oracle.quantize_kv_q8(kb.download(np.float32)))
+
+
+@pytest.mark.parametrize("kv", [KvType.F32, KvType.F16, KvType.Q8_0])
+@pytest.mark.parametrize("tokens,hq,hkv", [(170, 32, 8), (171, 32, 8), (1171, 5, 1), (1173, 5, 1)])
+def test_qk_norm_rope_store_rows_per_wave(kv, tokens, hq, hkv):
+    """Around 8192 rows a launch goes from one row per wave to four (171 * 48 and 1171 * 7 rows
+    are the first above, the last wave left with 1 or 3 rows): the same bits as the tokens in
+    chunks of at most 64."""
+    k = Kernels()
+    rng = oracle.Rng(67)
+    table = RopeTable(1e6, D, tokens)
+    x = [rng.vec(tokens * n * D, 3.0) for n in (hq, hkv, hkv)]
+    qn, kn = (DeviceBuffer.from_array(rng.vec(D, 1.5)) for _ in range(2))
+    row = kv.bytes(hkv * D)
+
+    def run(step):
+        q, kb, v = (DeviceBuffer.from_array(a) for a in x)
+        kc, vc = DeviceBuffer(tokens * row), DeviceBuffer(tokens * row)
+        for t in range(0, tokens, step):
+            n = min(step, tokens - t)
+            k.qk_norm_rope_store(kv, ((q, 4 * t * hq * D), (kb, 4 * t * hkv * D), (v, 4 * t * hkv * D)),
+                                 (qn, kn), 1e-6, table, ((kc, t * row), (vc, t * row)),
+                                 AttnShape(n, hq, hkv, D, t, kv))
+        synchronize()
+        return [b.download(np.uint8) for b in (q, kb, kc, vc)]
+
+    print(f"qkv rows per wave kv={kv.name_str} T={tokens} hq={hq}", flush=True)
+    for a, b in zip(run(tokens), run(64)):
+        assert np.array_equal(a, b)
