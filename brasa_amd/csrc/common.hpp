@@ -287,6 +287,31 @@ __device__ __forceinline__ void lds_dma4_s(const uint8_t* sbase, uint32_t voff,
         : "v"(voff), "s"(sbase), "s"(lds_wave_base)
         : "memory");
 }
+// 16- and 4-byte copies from per-lane 64-bit addresses (lane i writes lds + 16 i, lds + 4 i).
+__device__ __forceinline__ void lds_dma16_v(const uint8_t* src, uint32_t lds_wave_base) {
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 2\n\t"
+        "global_load_lds_dwordx4 %1, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(src), "s"(lds_wave_base)
+        : "memory");
+}
+__device__ __forceinline__ void lds_dma4(const uint8_t* src, uint32_t lds_wave_base) {
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 2\n\t"
+        "global_load_lds_dword %1, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(src), "s"(lds_wave_base)
+        : "memory");
+}
 // Device-coherent stores and loads (written through / read past the XCD's L2): a partial
 // stored by a workgroup on one XCD is then visible to the merging workgroup on any other.
 __device__ __forceinline__ void st_dev16(float* p, f32x4 v) {

@@ -1411,9 +1411,13 @@ decode_q8_kernel(DecodeArgs<NS> a) {
 
 
 // ---- q8_0 caches, GQA group 4: the LDS copies above, cheaper block math -------------------
-// decode_q8h_kernel: decode_q8_kernel's workgroup, grid, copies (K and V codes and scales into
-// the wave's LDS ring slots, block i + 1 issued once block i has landed) and split merge, with
-// block math that needs no V tile rewrite, no factor table and no hi / lo split of P.
+// decode_q8h_kernel: decode_q8_kernel's workgroup, grid and split merge, with block math that
+// needs no V tile rewrite, no factor table and no hi / lo split of P, on units of 16 keys (half a
+// 32-key block: a 128-key split feeds all eight waves, and a wave's last unit is half the math
+// after its data). A wave keeps one unit in flight: unit i + 1 is issued once unit i has landed.
+// More in flight only lengthens the memory system's queues (16K keys: 13.6 us a layer with one,
+// 15.1 with two, 15.5 with three; 32-key blocks, one in flight, 15.2; sixteen waves of two units
+// 15.4). 4097 keys 11.0 -> 9.3 us, 12000 13.9 -> 12.0, 32768 22.9 -> 20.5.
 // Lane l = (u = l / 16, c = l % 16), c = 4 gq + jh.
 //  * S^T = K Q^T on v_mfma_f32_16x16x32_f16, one k-step per 32-dim group t: the A operand is
 //    key c of the 16-key tile, dims 32 t + 8 u .. + 7 (codes exact in f16, read from LDS as in
@@ -1429,7 +1433,9 @@ decode_q8_kernel(DecodeArgs<NS> a) {
 //    touches fall in both halves of the banks). Accumulator e (0..7) holds, in lane (u, c),
 //    O[head 0..3][dim 32 gq + 8 jh + e] over the keys 4 u + r; the four u are summed at the
 //    wave's end.
-constexpr int kQ8hSlot = 2 * kQ8Codes + 2 * kBlock * 8;  // K codes, V codes, K scales, V scales
+constexpr int kQ8hCodes = kUnit * 128;                   // bytes of one tile's codes
+constexpr int kQ8hSlot = 2 * kQ8hCodes + 2 * kUnit * 8;  // K codes, V codes, K scales, V scales
+constexpr int kQ8hCopies = 5;                            // copy instructions of one unit
 
 template <int NS, int HPW, int W>
 __global__ void __launch_bounds__(64 * W)
@@ -1440,6 +1446,7 @@ decode_q8h_kernel(DecodeArgs<NS> a) {
     constexpr int KS = W / HPW;
     static_assert(W <= kMaxLdsWaves, "waves per workgroup");
     static_assert(finish_floats<G, W>() * 4 <= W * kRing * kQ8hSlot, "merge area in the ring");
+    static_assert(G * kDim * 4 <= kQ8hSlot, "Q in a ring slot");
     __shared__ __attribute__((aligned(16))) uint8_t s_slot[W][kRing][kQ8hSlot];
 
     const int rows = (a.ngroups + HPW - 1) / HPW;
@@ -1461,82 +1468,84 @@ decode_q8h_kernel(DecodeArgs<NS> a) {
     const int gq = c >> 2, jh = c & 3;
     const int uo = u & 1;
 
-    // the split's 32-key blocks interleaved with the other splits', as in decode_f16_kernel
+    // the split's 32-key blocks interleaved with the other splits', as in decode_f16_kernel, in
+    // units of 16 keys; the sequence's last block may hold one unit only
     const SplitBlocks sb = split_blocks(sd.lk, sd.splits, split);
     const int s1 = sd.lk;
-    const int nblk = sb.count;
-    const int bstride = sb.stride;
-    const int s0 = sb.first;
-    const int nb = (hg_ok && nblk > ks) ? (nblk - ks + KS - 1) / KS : 0;
+    const int nun = 2 * sb.count - (s1 - (sb.first + sb.stride * (sb.count - 1)) <= kUnit ? 1 : 0);
+    const int nb = (hg_ok && nun > ks) ? (nun - ks + KS - 1) / KS : 0;  // this wave's units
+    auto key_of = [&](int i) {
+        const int x = ks + KS * i;
+        return sb.first + sb.stride * (x >> 1) + kUnit * (x & 1);
+    };
     const size_t kstride = (size_t)a.hkv * RB;
     const uint8_t* kbase = sgpr_base(sd.k + (size_t)kh * RB);
     const uint8_t* vbase = sgpr_base(sd.v + (size_t)kh * RB);
 
-    u32x4 qr[8];
-    {
-        // column c: head h0 + jh; k-step t: dims 32 t + 8 u .. + 7
-        const uint8_t* qrow = reinterpret_cast<const uint8_t*>(qseq + (size_t)(h0 + jh) * kDim);
+    // Unit i -> slot i % 2: K codes (2 instructions of 8 rows, chunks swizzled), V codes (2), then
+    // one 4-byte instruction for the scales: lanes 0-31 the K scales (row lane / 2, dword lane % 2),
+    // lanes 32-63 the V scales
+    const int lr = lane >> 3, lc = lane & 7, sr = (lane & 31) >> 1;
+    const uint32_t soff = 128 + 4 * (lane & 1);
+    uint32_t off_k[2], off_v[2];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            qr[2 * t] = ld16_asm(qrow + 4 * (32 * t + 8 * u));
-            qr[2 * t + 1] = ld16_asm(qrow + 4 * (32 * t + 8 * u + 4));
-        }
-    }
-    // block i -> slot S, as decode_q8_kernel: K codes (4 instructions, 8 rows each, swizzled), V
-    // codes (4, swizzled), K scales, V scales (one 4-byte instruction each)
-    const int lr = lane >> 3, lc = lane & 7, sr = lane >> 1;
-    uint32_t off_k[4], off_v[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < 2; ++r) {
         const int rr = 8 * r + lr;
         off_k[r] = (uint32_t)(rr * kstride) + 16 * (lc ^ ((rr >> 1) & 7));
         off_v[r] = (uint32_t)(rr * kstride) + 16 * (lc ^ q8_vswz(rr));
     }
-    const uint32_t off_s = (uint32_t)(sr * kstride) + 128 + 4 * (lane & 1);
-    auto issue_at = [&](auto slot_c, int jb) {
+    const uint8_t* sbase = (lane < 32 ? sd.k : sd.v) + (size_t)kh * RB + soff;
+    auto issue = [&](auto slot_c, int i) {
         constexpr int S = decltype(slot_c)::value;
+        const int jb = key_of(i);
         const uint32_t sl = lds_addr(&s_slot[wave][S][0]);
         const uint8_t* kb = sgpr_offset(kbase, (size_t)jb * kstride);
         const uint8_t* vb = sgpr_offset(vbase, (size_t)jb * kstride);
-        if (jb + kBlock <= s1) {
+        if (jb + kUnit <= s1) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) lds_dma16_s(kb, off_k[r], sl + 1024 * r);
+            for (int r = 0; r < 2; ++r) lds_dma16_s(kb, off_k[r], sl + 1024 * r);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) lds_dma16_s(vb, off_v[r], sl + kQ8Codes + 1024 * r);
-            lds_dma4_s(kb, off_s, sl + 2 * kQ8Codes);
-            lds_dma4_s(vb, off_s, sl + 2 * kQ8Codes + 256);
+            for (int r = 0; r < 2; ++r) lds_dma16_s(vb, off_v[r], sl + kQ8hCodes + 1024 * r);
         } else {
             const int last = s1 - 1 - jb;  // rows past it read the last row again
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < 2; ++r) {
                 const int rr = 8 * r + lr;
                 const uint32_t rowo = (uint32_t)(min(rr, last) * kstride);
                 lds_dma16_s(kb, rowo + 16 * (lc ^ ((rr >> 1) & 7)), sl + 1024 * r);
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < 2; ++r) {
                 const int rr = 8 * r + lr;
                 const uint32_t rowo = (uint32_t)(min(rr, last) * kstride);
-                lds_dma16_s(vb, rowo + 16 * (lc ^ q8_vswz(rr)), sl + kQ8Codes + 1024 * r);
+                lds_dma16_s(vb, rowo + 16 * (lc ^ q8_vswz(rr)), sl + kQ8hCodes + 1024 * r);
             }
-            const uint32_t srow = (uint32_t)(min(sr, last) * kstride) + 128 + 4 * (lane & 1);
-            lds_dma4_s(kb, srow, sl + 2 * kQ8Codes);
-            lds_dma4_s(vb, srow, sl + 2 * kQ8Codes + 256);
         }
+        lds_dma4(sbase + (size_t)min(jb + sr, s1 - 1) * kstride, sl + 2 * kQ8hCodes);
     };
-    auto issue = [&](auto slot_c, int i) { issue_at(slot_c, s0 + bstride * (ks + KS * i)); };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
-    // one block in flight at the start (a wave without blocks copies the split's first one,
-    // never read), then one wait with a fixed count for the Q loads, as decode_q8_kernel
-    issue_at(I0{}, nb > 0 ? s0 + bstride * ks : s0);
-    wait_k<10>(qr);
+    // The group's Q (4 rows of 512 bytes) goes to slot 1 first, then unit 0 to slot 0; no register
+    // of the kernel is written by a load in flight, so the waits below are plain counts.
+    {
+        const uint32_t sl = lds_addr(&s_slot[wave][1][0]);
+        const uint8_t* q0 = reinterpret_cast<const uint8_t*>(qseq + (size_t)h0 * kDim);
+        lds_dma16_v(q0 + 16 * lane, sl);
+        lds_dma16_v(q0 + 1024 + 16 * lane, sl + 1024);
+    }
+    if (nb > 0) {
+        issue(I0{}, 0);
+        wait_vmcnt<kQ8hCopies>();
+    } else {
+        wait_vmcnt<0>();
+    }
 
     half8 qh[4], ql[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        const f32x4 q0 = __builtin_bit_cast(f32x4, qr[2 * t]);
-        const f32x4 q1 = __builtin_bit_cast(f32x4, qr[2 * t + 1]);
+        // column c: head h0 + jh; k-step t: dims 32 t + 8 u .. + 7
+        const f32x4* qp = reinterpret_cast<const f32x4*>(&s_slot[wave][1][0] + jh * 512 + 128 * t + 32 * u);
+        const f32x4 q0 = qp[0], q1 = qp[1];
         const float sc = a.scale * kLog2e;  // scores come out in the log2 domain
         const float x[8] = {as_f32(q0.x * sc), as_f32(q0.y * sc), as_f32(q0.z * sc),
                             as_f32(q0.w * sc), as_f32(q1.x * sc), as_f32(q1.y * sc),
@@ -1552,41 +1561,37 @@ decode_q8h_kernel(DecodeArgs<NS> a) {
 
     auto step = [&](auto slot_c, int i) {
         constexpr int S = decltype(slot_c)::value;
-        wait_vmcnt<0>();  // block i: the only copies in flight
+        wait_vmcnt<0>();  // unit i: the only copies in flight
         if (i + 1 < nb) {
-            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the other slot's reads returned
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): unit i - 1's (or Q's) reads returned
             asm volatile("" ::: "memory");
             issue(std::integral_constant<int, 1 - S>{}, i + 1);
         }
         if (i == 0) DECODE_STAMP(kStampFirstBlock);
         if (i + 1 == nb) DECODE_STAMP(kStampLastBlock);
-        const int jb = s0 + bstride * (ks + KS * i);
+        const int jb = key_of(i);
         const uint8_t* sl = &s_slot[wave][S][0];
-        const uint8_t* vco = sl + kQ8Codes;
-        const uint8_t* ksc = sl + 2 * kQ8Codes;
-        const uint8_t* vsc = sl + 2 * kQ8Codes + 256;
-        // this lane's V codes and V scales (keys 16 kt + 4 u + (r ^ uo)), read first: they return
-        // while S and the softmax are computed
-        u32x2 vw[2][4];
-        uint16_t vs[2][4];
+        const uint8_t* vco = sl + kQ8hCodes;
+        const uint8_t* ksc = sl + 2 * kQ8hCodes;
+        const uint8_t* vsc = ksc + kUnit * 8;
+        // this lane's V codes and V scales (keys 4 u + (r ^ uo)), read first: they return while S
+        // and the softmax are computed
+        u32x2 vw[4];
+        uint16_t vs[4];
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int R = 16 * kt + 4 * u + (r ^ uo);
-                vw[kt][r] = *reinterpret_cast<const u32x2*>(vco + R * 128 + 16 * ((c >> 1) ^ q8_vswz(R)) + 8 * (c & 1));
-                vs[kt][r] = *reinterpret_cast<const uint16_t*>(vsc + R * 8 + 2 * gq);
-            }
+        for (int r = 0; r < 4; ++r) {
+            const int R = 4 * u + (r ^ uo);
+            vw[r] = *reinterpret_cast<const u32x2*>(vco + R * 128 + 16 * ((c >> 1) ^ q8_vswz(R)) + 8 * (c & 1));
+            vs[r] = *reinterpret_cast<const uint16_t*>(vsc + R * 8 + 2 * gq);
+        }
         // S^T: per 32-dim group t two chained MFMAs (Q hi, Q lo), scaled by the row's group scale
-        float x[2][4];
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            const int r16 = 16 * kt + c;
+        float x[4];
+        {
             f32x4 part[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int L = 2 * t + (u >> 1);
-                const u32x2 kc = *reinterpret_cast<const u32x2*>(sl + r16 * 128 + 16 * (L ^ ((r16 >> 1) & 7)) + 8 * (u & 1));
+                const u32x2 kc = *reinterpret_cast<const u32x2*>(sl + c * 128 + 16 * (L ^ ((c >> 1) & 7)) + 8 * (u & 1));
                 uint32_t l0, g0, l1, g1;
                 codes4_to_f16(kc.x, l0, g0);
                 codes4_to_f16(kc.y, l1, g1);
@@ -1594,28 +1599,21 @@ decode_q8h_kernel(DecodeArgs<NS> a) {
                 part[t] = mfma16(kf, ql[t], mfma16(kf, qh[t], f32x4{0.0f, 0.0f, 0.0f, 0.0f}));
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {  // scales of S row 16 kt + 4 u + r
-                const u32x2 sw = *reinterpret_cast<const u32x2*>(ksc + (16 * kt + 4 * u + r) * 8);
+            for (int r = 0; r < 4; ++r) {  // scales of S row 4 u + r
+                const u32x2 sw = *reinterpret_cast<const u32x2*>(ksc + (4 * u + r) * 8);
                 float v = fmaf(part[0][r], h2f((uint16_t)(sw.x & 0xffffu)), 0.0f);  // one mixed FMA
                 v = fmaf(part[1][r], h2f((uint16_t)(sw.x >> 16)), v);
                 v = fmaf(part[2][r], h2f((uint16_t)(sw.y & 0xffffu)), v);
                 v = fmaf(part[3][r], h2f((uint16_t)(sw.y >> 16)), v);
-                x[kt][r] = v;
+                x[r] = v;
             }
         }
-        if (jb + kBlock > s1) {  // the sequence's last block: keys past its end get -inf
+        if (jb + kUnit > s1) {  // the sequence's last unit: keys past its end get -inf
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (jb + 16 * kt + 4 * u + r >= s1) x[kt][r] = -INFINITY;
+            for (int r = 0; r < 4; ++r)
+                if (jb + 4 * u + r >= s1) x[r] = -INFINITY;
         }
-        float bm = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) bm = fmaxf(bm, x[kt][r]);
-        bm = max_rows(bm);
+        const float bm = max_rows(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
         if (__builtin_amdgcn_ballot_w64(bm > mref + kLazyRescale) != 0) {
             const float mn = fmaxf(mref, bm);
             const float alpha = __builtin_amdgcn_exp2f(mref - mn);  // of head jh
@@ -1628,38 +1626,33 @@ decode_q8h_kernel(DecodeArgs<NS> a) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[e] *= ah;
         }
-        float p[2][4];
+        float p[4];
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                p[kt][r] = __builtin_amdgcn_exp2f(x[kt][r] - mref);
-                lsum += p[kt][r];
-            }
+        for (int r = 0; r < 4; ++r) {
+            p[r] = __builtin_amdgcn_exp2f(x[r] - mref);
+            lsum += p[r];
+        }
         // O += P V: the key of step r is 4 u + (r ^ uo), its p picked from the lane's own four
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int r = 0; r < 4; ++r) {
+            const float pk = uo ? p[r ^ 1] : p[r];
+            const float av = fmaf(pk, h2f(vs[r]), 0.0f);  // one mixed FMA
+            const u32x2 w = vw[r];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float pk = uo ? p[kt][r ^ 1] : p[kt][r];
-                const float av = fmaf(pk, h2f(vs[kt][r]), 0.0f);  // one mixed FMA
-                const u32x2 w = vw[kt][r];
+            for (int e = 0; e < 4; ++e)
+                acc[e] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                    av, (float)(int8_t)(w.x >> (8 * e)), acc[e], 0, 0, 0);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    acc[e] = __builtin_amdgcn_mfma_f32_4x4x1f32(
-                        av, (float)(int8_t)(w.x >> (8 * e)), acc[e], 0, 0, 0);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    acc[4 + e] = __builtin_amdgcn_mfma_f32_4x4x1f32(
-                        av, (float)(int8_t)(w.y >> (8 * e)), acc[4 + e], 0, 0, 0);
-            }
+            for (int e = 0; e < 4; ++e)
+                acc[4 + e] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                    av, (float)(int8_t)(w.y >> (8 * e)), acc[4 + e], 0, 0, 0);
+        }
     };
     for (int i0 = 0; i0 < nb; i0 += kRing) {
         step(I0{}, i0);
         if (i0 + 1 >= nb) break;
         step(I1{}, i0 + 1);
     }
-    wait_vmcnt<0>();  // copies of a wave without blocks land before the LDS is reused below
 
     // ---- the split's end: sum the key quarters u, lane (u, c) keeps head u ------------------
     lsum = sum_rows(lsum);

@@ -72,17 +72,18 @@ def test_decode_other_groups(kv):
         assert w <= 1e-5, (hq, w)
 
 
-@pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 8), (32, 8), (64, 8)])
-def test_decode_f32_unit_edges(hq, hkv):
-    """The f32 kernel at the edges of its 16-key units, 32-key blocks and 128-key splits, for one
-    to eight heads per group. Every product and sum is f32: 4096 terms of random sign keep well
-    under 2e-6 of max|v| (measured 2-5e-7)."""
+@pytest.mark.parametrize("kv,hq,hkv", [(KvType.F32, 8, 8), (KvType.F32, 16, 8), (KvType.F32, 32, 8),
+                                       (KvType.F32, 64, 8), (KvType.Q8_0, 32, 8)])
+def test_decode_unit_edges(kv, hq, hkv):
+    """The f32 kernel, for one to eight heads per group, and the q8_0 group-4 kernel at the edges
+    of their 16-key units, 32-key blocks and 128-key splits. Sums of up to 4096 terms of random
+    sign in f32, on exact products, keep well under 2e-6 of max|v| (measured 2-5e-7)."""
     k = Kernels()
     rng = oracle.Rng(37)
     for lk in [1, 15, 16, 17, 31, 32, 33, 48, 49, 127, 129, 144, 145, 1039, 4081]:
         q = rng.vec(hq * DIM, 2.0)
-        cache = KvPair(KvType.F32, rng.vec(lk * hkv * DIM, 2.0), rng.vec(lk * hkv * DIM, 3.0))
-        _say(f"decode f32 edges hq={hq} lk={lk}")
+        cache = KvPair(kv, rng.vec(lk * hkv * DIM, 2.0), rng.vec(lk * hkv * DIM, 3.0))
+        _say(f"decode unit edges kv={kv.name_str} hq={hq} lk={lk}")
         got = run_decode(k, "lanes", q, cache, hq, hkv, lk - 1)
         want, vmax = oracle.attention(q, cache.k, cache.v, 1, hq, hkv, DIM, lk - 1)
         w = oracle.worst(got, want, vmax)
