@@ -530,20 +530,21 @@ __device__ __forceinline__ void finish_split(const DecodeArgs<NS>& a, const SeqD
 // ---- f16 caches: every load explicit --------------------------------------------------------
 // Workgroup = HPW adjacent head groups x one split of sd.chunk keys, W wave64; wave w works for
 // head group w % HPW and walks the 32-key blocks ks, ks + KS, ... of the split (ks = w / HPW,
-// KS = W / HPW), so at any time the workgroup reads HPW adjacent KV heads' rows. A wave keeps up to kRing blocks in flight: K rows go
-// from HBM into registers (the MFMA A operand), V rows HBM -> LDS (global_load_lds_dwordx4, read
-// transposed by ds_read_tr16_b64), Q into registers. Every vector-memory instruction of the
-// block loop is inline asm, issued in a fixed order, so each wait is an exact count: block i is
-// ready when the blocks issued after it (at most kRing - 1, 16 instructions each) are the only
-// ones pending. The wait names the registers it guards as operands, so no use of them can be
-// scheduled above it. Block i + kRing is issued into block i's ring slot once block i has been
-// computed.
+// KS = W / HPW), so at any time the workgroup reads HPW adjacent KV heads' rows. K rows go from HBM
+// into registers (the MFMA A operand), V rows HBM -> LDS (global_load_lds_dwordx4, read transposed
+// by ds_read_tr16_b64), Q HBM -> LDS. Every vector-memory instruction of the block loop is inline
+// asm. A wave keeps one block in flight: block i + 1 is issued into the other ring slot once block
+// i has landed; two from the start only lengthen the memory system's queues, and every wave's
+// first block lands later (16K keys: 16.1 us a layer with one, 16.45 with two; 1000 keys 7.25,
+// 7.9). Four heads per workgroup, the layout of large batches, keep two (59.0 us against 59.35 for
+// 8 sequences of 1024 to 16384 keys). The wait names the K registers it guards as operands, so no
+// use of them can be scheduled above it.
 // Softmax: columns c < G hold the hi halves of the split Q / P operands, the partner columns
 // (col_is_lo) the lo halves; one DPP exchange adds them (the same bits in both lanes). Only the
 // sequence's last block masks keys past its end. The running max is lazy: the
 // reference point moves only when a block's max exceeds it by more than 2^8, so most blocks skip
 // the rescale of O.
-constexpr int kRing = 2;                    // blocks in flight per wave (16 instructions each)
+constexpr int kRing = 2;                    // ring slots per wave
 constexpr int kMaxLdsWaves = 8;
 constexpr int kTileHalves = kBlock * kDim;  // one 32 x 128 f16 tile = 8 KB
 constexpr float kLazyRescale = 8.0f;        // log2 of the largest P value before a rescale
@@ -596,6 +597,8 @@ decode_f16_kernel(DecodeArgs<NS> a) {
     constexpr int kFin = finish_floats<G, W>();
     constexpr bool kSepFin = W * kRing * kTileHalves * 2 + kFin * 4 <= 160 * 1024;
     __shared__ __attribute__((aligned(16))) float s_fin[kSepFin ? kFin : 1];
+    constexpr bool kTwo = HPW == 4;  // two blocks in flight, else one
+    static_assert(!kTwo || kSepFin, "Q beside the ring");
 
     // grid: (split column, row of HPW head groups), rows innermost
     const int rows = (a.ngroups + HPW - 1) / HPW;
@@ -633,15 +636,19 @@ decode_f16_kernel(DecodeArgs<NS> a) {
     const uint8_t* kbase = sd.k + (size_t)kh * RB;
     const uint8_t* vbase = sd.v + (size_t)kh * RB;
 
-    // Q rows of this lane's column (dims 32 t + 8 u .. + 8 for t < 4), loaded first
-    u32x4 qr[8];
+    // The group's Q rows go to LDS first: copied, not loaded, so that no register but K's waits on
+    // memory. To the wave's V slot 1, free until block 1 is issued, or (two in flight) to the merge
+    // area, at the wave's own accumulators there (one head: past all of them)
+    constexpr int kQCopies = G > 2 ? G / 2 : 1;
+    const float* s_q = kTwo ? s_fin + (G == 1 ? 2 * kDim * (W + wave) : kDim * G * wave)
+                            : reinterpret_cast<const float*>(&s_v[wave][1][0]);
+    static_assert(G != 1 || !kSepFin || (2 * kDim * 2 * W <= kFin && W * (kDim + 2) <= 2 * kDim * W), "Q of one head");
     {
-        const uint8_t* qrow = reinterpret_cast<const uint8_t*>(qseq + (size_t)(h0 + col_head<G>(c16)) * kDim);
+        const uint32_t sl = __builtin_amdgcn_readfirstlane(lds_addr(s_q));
+        const uint8_t* q0 = reinterpret_cast<const uint8_t*>(qseq + (size_t)h0 * kDim);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            qr[2 * t] = ld16_asm(qrow + 4 * (32 * t + 8 * u));
-            qr[2 * t + 1] = ld16_asm(qrow + 4 * (32 * t + 8 * u + 4));
-        }
+        for (int r = 0; r < kQCopies; ++r)  // (one head: lanes 32-63 copy the row again)
+            lds_dma16_v(q0 + 1024 * r + 16 * (G == 1 ? lane & 31 : lane), sl + 1024 * r);
     }
     u32x4 kr[kRing][8];
     // block i of this wave -> ring slot S: 8 K loads (tile row 16 kt + c16, dims 32 t + 8 u in
@@ -665,12 +672,13 @@ decode_f16_kernel(DecodeArgs<NS> a) {
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     if (nb > 0) issue(I0{}, 0);
-    if (nb > 1) issue(I1{}, 1);
-    // Q was issued first: it has landed when at most the blocks' instructions are pending
-    switch (min(nb, kRing)) {
-        case 2: wait_k<32>(qr); break;
-        case 1: wait_k<16>(qr); break;
-        default: wait_k<0>(qr); break;
+    if (kTwo && nb > 1) {  // then wait for Q
+        issue(I1{}, 1);
+        wait_vmcnt<32>();
+    } else if (nb > 0) {
+        wait_vmcnt<16>();
+    } else {
+        wait_vmcnt<0>();
     }
 
     // ---- Q^T B-operand: k-step t holds dims 32 t + 8 u + j; column c < G: head h0 + c, hi half;
@@ -680,8 +688,8 @@ decode_f16_kernel(DecodeArgs<NS> a) {
         const float sc = (colq || col_lo) ? a.scale * kLog2e : 0.0f;  // scores in the log2 domain
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const f32x4 q0 = __builtin_bit_cast(f32x4, qr[2 * t]);
-            const f32x4 q1 = __builtin_bit_cast(f32x4, qr[2 * t + 1]);
+            const f32x4* qp = reinterpret_cast<const f32x4*>(s_q + kDim * col_head<G>(c16) + 32 * t + 8 * u);
+            const f32x4 q0 = qp[0], q1 = qp[1];
             const float x[8] = {as_f32(q0.x * sc), as_f32(q0.y * sc), as_f32(q0.z * sc),
                                 as_f32(q0.w * sc), as_f32(q1.x * sc), as_f32(q1.y * sc),
                                 as_f32(q1.z * sc), as_f32(q1.w * sc)};  // f32: q * (scale log2 e)
@@ -701,9 +709,13 @@ decode_f16_kernel(DecodeArgs<NS> a) {
     // One step computes block i from ring slot S and refills the slot with block i + kRing.
     auto step = [&](auto slot_c, int i) {
         constexpr int S = decltype(slot_c)::value;
-        // block i's 16 instructions were followed by those of the block after it in the ring
-        if (i + 1 < nb) wait_k<16>(kr[S]);
+        if (kTwo && i + 1 < nb) wait_k<16>(kr[S]);
         else wait_k<0>(kr[S]);
+        if (!kTwo && i + 1 < nb) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): block i - 1's (or Q's) reads returned
+            asm volatile("" ::: "memory");
+            issue(std::integral_constant<int, 1 - S>{}, i + 1);
+        }
         if (i == 0) DECODE_STAMP(kStampFirstBlock);
         if (i + 1 == nb) DECODE_STAMP(kStampLastBlock);
         const int jb = s0 + bstride * (ks + KS * i);
@@ -766,7 +778,7 @@ decode_f16_kernel(DecodeArgs<NS> a) {
         // O^T += V^T P^T; P^T slot j of lane (c, u) is key j < 4 ? 4u + j : 16 + 4u + j - 4
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) acc[dt] = mfma16(va[dt], pb, acc[dt]);
-        if (i + kRing < nb) {
+        if (kTwo && i + kRing < nb) {
             // the slot's LDS reads have returned (their values fed the MFMAs above) before the
             // next block's copies into it are issued
             __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
@@ -813,7 +825,8 @@ decode_f16_kernel(DecodeArgs<NS> a) {
 // Workgroup = one head group x one split, W wave64; a wave walks units of 16 keys (half a 32-key
 // block, so a 128-key split still feeds 8 waves), w, w + W, ... A unit is 16 loads of 16 bytes per
 // lane, K and V straight into registers, each instruction covering 4 whole rows; a wave keeps
-// two units in flight with exact waits, as decode_f16_kernel. Lane l = 16 u + c = 4 b + j.
+// two units in flight, with exact waits (one: the same within 1 %, 4097 keys 11.35 -> 11.6 us).
+// Lane l = 16 u + c = 4 b + j.
 //  * S: block b takes dims 8 b .. 8 b + 7, A = q of head j (4 lanes: 4 heads), B = K of key
 //    4 t + j: D of lane (b, j) is the partial score of key 4 t + j for the 4 heads. The 16 blocks
 //    are summed by permlane swaps that leave tile t = u in row u, then by two DPP rotations in
