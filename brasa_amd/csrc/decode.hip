@@ -706,7 +706,8 @@ decode_f16_kernel(DecodeArgs<NS> a) {
     for (int dt = 0; dt < 8; ++dt) acc[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const int trc = (c16 & 3), trj = (c16 >> 2);
 
-    // One step computes block i from ring slot S and refills the slot with block i + kRing.
+    // One step computes block i from ring slot S; block i + 1 is issued before it, or (kTwo) block
+    // i + 2 into this slot after it.
     auto step = [&](auto slot_c, int i) {
         constexpr int S = decltype(slot_c)::value;
         if (kTwo && i + 1 < nb) wait_k<16>(kr[S]);

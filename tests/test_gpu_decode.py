@@ -73,10 +73,12 @@ def test_decode_other_groups(kv):
 
 
 @pytest.mark.parametrize("kv,hq,hkv", [(KvType.F32, 8, 8), (KvType.F32, 16, 8), (KvType.F32, 32, 8),
-                                       (KvType.F32, 64, 8), (KvType.Q8_0, 32, 8)])
+                                       (KvType.F32, 64, 8), (KvType.Q8_0, 32, 8),
+                                       (KvType.F16, 8, 8), (KvType.F16, 16, 8), (KvType.F16, 32, 8),
+                                       (KvType.F16, 64, 8)])
 def test_decode_unit_edges(kv, hq, hkv):
-    """The f32 kernel, for one to eight heads per group, and the q8_0 group-4 kernel at the edges
-    of their 16-key units, 32-key blocks and 128-key splits. Sums of up to 4096 terms of random
+    """The f32 and f16 kernels, for one to eight heads per group, and the q8_0 group-4 kernel at the
+    edges of their 16-key units, 32-key blocks and 128-key splits. Sums of up to 4096 terms of random
     sign in f32, on exact products, keep well under 2e-6 of max|v| (measured 2-5e-7)."""
     k = Kernels()
     rng = oracle.Rng(37)
@@ -88,6 +90,29 @@ def test_decode_unit_edges(kv, hq, hkv):
         want, vmax = oracle.attention(q, cache.k, cache.v, 1, hq, hkv, DIM, lk - 1)
         w = oracle.worst(got, want, vmax)
         assert w <= 2e-6, (lk, w)
+
+
+@pytest.mark.parametrize("kv,hq", [(KvType.F16, 8), (KvType.F16, 32), (KvType.Q8_0, 32),
+                                   (KvType.F32, 32)])
+def test_decode_q_at_any_float(kv, hq):
+    """Q at any f32 address (copied 16 bytes a lane): the same bits as 16-byte aligned, without
+    blocks for some waves, with one each and with several."""
+    k = Kernels()
+    rng = oracle.Rng(41)
+    for lk in [5, 130, 1500]:
+        q = rng.vec(hq * DIM, 2.0)
+        cache = KvPair(kv, rng.vec(lk * HKV * DIM, 2.0), rng.vec(lk * HKV * DIM, 3.0))
+        want = run_decode(k, "lanes", q, cache, hq, HKV, lk - 1)
+        for off in (1, 2, 3):
+            _say(f"decode q at a float kv={kv.name_str} hq={hq} lk={lk} off={off}")
+            buf = DeviceBuffer.from_array(np.concatenate([np.zeros(off, np.float32), q,
+                                                          np.zeros(4, np.float32)]))
+            part = DeviceBuffer(4 * decode_partials_len(hq, lk))
+            o = DeviceBuffer(hq * DIM * 4)
+            k.decode_attention_lanes(buf.ptr + 4 * off, cache.kbuf, cache.vbuf, part, o,
+                                     AttnShape(1, hq, HKV, DIM, lk - 1, kv), out=OutDType.F32)
+            synchronize()
+            assert np.array_equal(o.download(np.float32).reshape(hq, DIM), want), (lk, off)
 
 
 @pytest.mark.parametrize("kv", KVS)
