@@ -1213,7 +1213,9 @@ prefill_q8_kernel4(PrefillArgs a) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
         }
-        const float mb = m_used * kLog2e;
+        // a column without a key so far (a key part's stages can all lie past a column's query) has
+        // m = -inf and every s = -inf: P = 2^(-inf - 0) = 0, where -inf - -inf would make NaN
+        const float mb = m_used == -INFINITY ? 0.0f : m_used * kLog2e;
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             if (b >= nsub) break;

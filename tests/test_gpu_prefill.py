@@ -497,6 +497,34 @@ def test_flash_exact_split_workspace():
         assert size < need or np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("hq,hkv,tokens,pos0", [(4, 1, 137, 56), (2, 1, 200, 56), (1, 1, 73, 120),
+                                                (4, 1, 383, 0)])
+def test_flash_q8_key_parts_past_a_query(hq, hkv, tokens, pos0):
+    """q8_0 key parts that start past some queries of a wave, or hold no key of a query tile at
+    all: such a column's state is (m, l, O) = (-inf, 0, 0) in the workspace, with no NaN that a
+    merge would have to leave out, and the output holds the bars."""
+    k = Kernels()
+    rng = oracle.Rng(109 + tokens)
+    cap = (pos0 + tokens + 63) // 64 * 64
+    q = rng.vec(tokens * hq * DIM, 2.0)
+    cache = KvPair(KvType.Q8_0, rng.vec(cap * hkv * DIM, 2.0), rng.vec(cap * hkv * DIM, 3.0))
+    shape = AttnShape(tokens, hq, hkv, DIM, pos0, KvType.Q8_0)
+    F16 = PrefillPrecision.F16
+    need = Kernels.flash_attention_workspace_len(shape, F16)
+    assert need > 0
+    gq, ws = DeviceBuffer.from_array(q), DeviceBuffer(need)
+    o = DeviceBuffer(tokens * hq * DIM * 2)
+    ws.fill(0)  # (states of padding columns are not written)
+    _say(f"prefill q8_0 parts past a query hq={hq} hkv={hkv} T={tokens} pos0={pos0}")
+    k.flash_attention_ws(gq, cache.kbuf, cache.vbuf, o, shape, F16, ws, need)
+    synchronize()
+    state = ws.download(np.float32)
+    assert np.isneginf(state).any() and not np.isnan(state).any()
+    ref16, _ = oracle.attention(q, cache.k, cache.v, tokens, hq, hkv, DIM, pos0, q16=True)
+    a, r = bars(oracle.f16_to_f32(o.download(np.uint16).reshape(tokens, hq, DIM)), ref16)
+    assert a <= 2e-3 and r <= 1e-2, (a, r)
+
+
 Q8_RANGE_CASES = [(9, 2500, "k_large"), (40, 4000, "k_large"), (64, 500, "k_large"), (64, 500, "v_large"), (64, 500, "tiny"),
                   (384, 0, "k_large"), (384, 0, "v_large"), (384, 0, "tiny")]
 
