@@ -1817,10 +1817,12 @@ prefill_merge_kernel(PrefillArgs a) {
         float Lr = 0.0f;
 #pragma unroll
         for (int p = 0; p < kPer; ++p) {
-            const bool ok = p0 + p < a.kparts && ml[p][0] != -INFINITY;
-            const float w = ok ? __builtin_amdgcn_exp2f((ml[p][0] - Mr) * kLog2e) : 0.0f;
-            Ar += w * (ok ? av[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-            Lr += w * (ok ? ml[p][1] : 0.0f);
+            // A part that saw no key of the column has (m, l, O) = (-inf, 0, 0) and weight 0. One
+            // whose scores are all NaN has m = -inf too: 0 * NaN keeps its NaN in the result
+            const bool in = p0 + p < a.kparts;
+            const float w = ml[p][0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((ml[p][0] - Mr) * kLog2e);
+            Ar += in ? w * av[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            Lr += in ? w * ml[p][1] : 0.0f;
         }
         const float Mn = fmaxf(M, Mr);
         const float w0 = (M == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((M - Mn) * kLog2e);

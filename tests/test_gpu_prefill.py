@@ -23,6 +23,7 @@ from gpu_util import DIM, HKV, HQ, KvPair, bars
 pytestmark = pytest.mark.gpu
 
 KVS = [KvType.F32, KvType.F16, KvType.Q8_0]
+PART_BYTES = 4 * 17 * 64 * 16  # workspace of one key part of a query tile
 # worst_f16 of the F16 hot path (P rounded to f16; q8_0 values as f16(code * scale)) against the
 # reference's attention_q16 over the exact cache values, on the reference's own case matrix:
 # measured 1.68e-4 (f32 cache), 1.87e-4 (f16), 5.34e-4 (q8_0), held with ~1.3x margin (the
@@ -523,6 +524,47 @@ def test_flash_q8_key_parts_past_a_query(hq, hkv, tokens, pos0):
     ref16, _ = oracle.attention(q, cache.k, cache.v, tokens, hq, hkv, DIM, pos0, q16=True)
     a, r = bars(oracle.f16_to_f32(o.download(np.uint16).reshape(tokens, hq, DIM)), ref16)
     assert a <= 2e-3 and r <= 1e-2, (a, r)
+
+
+@pytest.mark.parametrize("kv,precision,tokens,pos0", [
+    (KvType.F16, "F16", 45, 7001), (KvType.F16, "F16_PF32", 9, 7000), (KvType.F16, "F16", 150, 3000),
+    (KvType.F16, "F32", 40, 3000), (KvType.F32, "F32", 45, 7001), (KvType.F32, "F16", 40, 3000),
+    (KvType.Q8_0, "F16", 30, 4000), (KvType.Q8_0, "F16", 45, 7001), (KvType.Q8_0, "F32", 40, 3000)])
+def test_flash_nan_keys_of_whole_parts(kv, precision, tokens, pos0):
+    """NaN keys that fill whole key parts of a split call (one KV head, up to the boundary in the
+    middle of the first query tile's parts): every output of that head's query heads is NaN, as
+    without a split, and the other heads' bits are those of the clean cache. (q8_0: NaN scales; 150
+    tokens after 3000 is merged by the last part to arrive, the others by a launch of its own.)"""
+    synchronize()
+    assert lib().brasa_release_workspaces() == 0
+    prec = PrefillPrecision[precision]
+    need = Kernels.flash_attention_workspace_len(AttnShape(tokens, HQ, HKV, DIM, pos0, kv), prec)
+    cap = (pos0 + tokens + 63) // 64 * 64
+    if (kv, precision, tokens) == (KvType.Q8_0, "F16", 45):
+        need -= cap * HKV * DIM * 2 * 2  # the rows staged as f16
+    parts = need // (-(-tokens // 32) * HKV * PART_BYTES)
+    stage = 32 if precision == "F32" or kv == KvType.F32 else 64
+    nan_keys = -(-(pos0 + min(tokens, 32)) // stage) * (parts // 2) // parts * stage
+    assert parts > 1 and nan_keys > 0
+    k = Kernels()
+    rng = oracle.Rng(113 + tokens)
+    q = rng.vec(tokens * HQ * DIM, 2.0)
+    cache = KvPair(kv, rng.vec(cap * HKV * DIM, 2.0), rng.vec(cap * HKV * DIM, 3.0))
+    _say(f"prefill NaN keys kv={kv.name_str} {precision} T={tokens} pos0={pos0}")
+    clean = run_prefill(k, q, cache, tokens, HQ, HKV, pos0, prec)
+    rows = cache.kbuf.download(np.uint8).reshape(cap, HKV, -1)
+    bad = rows[:nan_keys, 3]
+    if kv == KvType.Q8_0:
+        bad[:, DIM:] = np.full((len(bad), 4), np.nan, np.float16).view(np.uint8)
+    else:
+        t = np.float16 if kv == KvType.F16 else np.float32
+        bad[:] = np.full((len(bad), DIM), np.nan, t).view(np.uint8)
+    cache.kbuf.upload(rows)
+    o = run_prefill(k, q, cache, tokens, HQ, HKV, pos0, prec).reshape(tokens, HKV, -1)
+    nan = np.isnan(o.view(np.float16) if o.dtype == np.uint16 else o)
+    assert nan[:, 3].all() and not np.delete(nan, 3, 1).any()
+    if kv != KvType.Q8_0 or precision != "F16":  # (a NaN scale takes the call's exact path)
+        assert np.array_equal(np.delete(o, 3, 1), np.delete(clean.reshape(o.shape), 3, 1))
 
 
 Q8_RANGE_CASES = [(9, 2500, "k_large"), (40, 4000, "k_large"), (64, 500, "k_large"), (64, 500, "v_large"), (64, 500, "tiny"),
