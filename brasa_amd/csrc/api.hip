@@ -268,7 +268,7 @@ int brasa_flash_attention_ws(const float* q, const void* k, const void* v, void*
     if (st != BRASA_OK) return st;
     if (s.tokens == 0) return BRASA_OK;
     if (!q || !k || !v || !o) return set_error(BRASA_ERR_ARG, "flash_attention: null pointer");
-    // (a split that only speeds the exact precisions up is left out of a smaller workspace)
+    // (a split that only makes the call faster is left out of a smaller workspace)
     size_t need = 0;
     prefill_workspace_len((int)s.tokens, (int)s.hq, (int)s.hkv, (int)s.pos0, s.kv, precision, &need);
     if (workspace_len < need || (need > 0 && !workspace))

@@ -1896,8 +1896,7 @@ struct PfCtx {
     size_t used = 0;
     bool measure = false;
     size_t need = 0;
-    size_t required = 0;    // without the parts of the plan a call can do without
-    bool optional = false;  // what is taken from now on is such a part
+    size_t required = 0;  // of `need`, without what a call with a smaller workspace leaves out
     unsigned* ctr = nullptr;
     unsigned* taint = nullptr;
     unsigned tag = 0;
@@ -1909,11 +1908,12 @@ struct PfCtx {
     int parts = 1;
 
     size_t room() const { return ws ? ws_len - used : 0; }
-    void* take(size_t bytes) {
+    // (must: the share of it that goes into `required`)
+    void* take(size_t bytes, size_t must) {
         bytes = (bytes + 255) / 256 * 256;
         if (measure) {
             need += bytes;
-            if (!optional) required += bytes;
+            required += (must + 255) / 256 * 256;
             return reinterpret_cast<void*>(static_cast<uintptr_t>(256));  // never dereferenced
         }
         if (!ws || used + bytes > ws_len) return nullptr;
@@ -1928,6 +1928,14 @@ struct KeySplit {
     int parts;
     bool two_step;  // merged by a launch of its own
 };
+// The split whose partials the caller's workspace of an F16 or F16_PF32 call has to hold: doubled
+// while the launch fills at most half of `slots` and its parts keep 16 tiles. What the rules below
+// split beyond it only makes the call faster, and is left out of a smaller workspace.
+int required_parts(long long wgs, int keys, int slots) {
+    int parts = 1;
+    while (parts < 8 && wgs * parts * 2 <= slots && keys / (kTile * parts * 2) >= 16) parts *= 2;
+    return parts;
+}
 // A split pays where the launch leaves CUs idle and a tile's keys are long. Its parts' partials
 // are 64 KB per part and tile; with few query tiles a launch of their own merges them, spread
 // over the chip, and the time left, tiles / P for the keys plus wgs * P for the partials, is
@@ -1950,15 +1958,15 @@ KeySplit split_in_kernel(long long wgs, int tiles, int slots) {
 }
 constexpr int kFewTiles = 16;  // query tiles up to which the merge is a launch of its own
 int key_tiles(int keys) { return (keys + kTile - 1) / kTile; }
-// the two-group f16 kernel, one workgroup per CU
-KeySplit key_split_f16(long long wgs, int keys) {
+// the two-group f16 kernel, one workgroup per CU; `most` parts
+KeySplit key_split_f16(long long wgs, int keys, int most) {
     const int tiles = key_tiles(keys);
     if (tiles < 12) return KeySplit{1, false};
-    if (wgs <= kFewTiles) return split_two_step(4.5, wgs, tiles, 256, 16);
+    if (wgs <= kFewTiles) return split_two_step(4.5, wgs, tiles, 256, most);
     const KeySplit k = split_in_kernel(wgs, tiles, 256);
     // more than 6 parts: the own launch once the keys are long enough to pay for it
     if (k.parts <= 6) return k;
-    return tiles >= 64 ? KeySplit{(int)(256 / wgs), true} : KeySplit{6, false};
+    return tiles >= 64 ? KeySplit{(int)std::min<long long>(256 / wgs, most), true} : KeySplit{6, false};
 }
 // prefill_q8_kernel4, two workgroups per CU. The merge launch also reads the range flag, in
 // place of the launch of prefill_exact_kernel an unsplit call needs, so it pays from few tiles on
@@ -1978,6 +1986,12 @@ KeySplit key_split_exact(long long wgs, int keys) {
     return split_two_step(9.0, wgs, tiles, 256, std::min(tiles, kMaxKeyParts));
 }
 
+// f16 rows staged from a q8_0 cache: no more parts than required_parts can ask for, so that a
+// workspace that holds the staging and 8 parts is the whole one (64 tokens after 8192, which ask
+// for 8: 41.0 us; 13 parts, as the f16 rule has it, 38.1; 45 after 7001 36.1 and 34.6 with 12)
+constexpr int kStagedParts = 8;
+constexpr int kF16Parts = 16;
+
 // parts within the limits of the workspace layout and the counter slot, else 1
 int clamp_parts(int parts, long long wgs) {
     return (parts < 1 || parts > kMaxKeyParts || wgs * 4 * 16 > kPfSlotWords) ? 1 : parts;
@@ -1987,17 +2001,17 @@ int clamp_parts(int parts, long long wgs) {
 // parts' partials in the call's workspace), merged by the last part to arrive (two_step false:
 // the stream's arrival counters) or by a launch of prefill_merge_kernel. Returns 1 when the
 // workspace or the counters are missing: the caller then launches unsplit. With room for fewer
-// parts only, it splits over those.
+// parts only, it splits over those; a caller's workspace has to hold `must` of them (1: none).
 template <int HW, bool OF32, bool GATED, typename K>
 int launch_split(PfCtx& c, K kernel, const char* name, PrefillArgs b, long long wgs, int parts,
-                 bool two_step, int threads) {
+                 int must, bool two_step, int threads) {
     const size_t unit = (size_t)wgs * kKeyPartFloats * sizeof(float);
     if (!c.measure) {
         if (!c.ctr) return 1;
         parts = (int)std::min<size_t>(parts, c.room() / unit);
         if (parts < 2) return 1;
     }
-    void* ws = c.take(unit * parts);
+    void* ws = c.take(unit * parts, must > 1 ? unit * std::min(parts, must) : 0);
     if (c.measure) return BRASA_OK;
     b.pair = 0;
     b.kparts = parts;
@@ -2072,9 +2086,8 @@ int launch(PfCtx& c, const PrefillArgs& a) {
     const long long wgs = (long long)(a.hq / HW) * a.ntiles;
     const KeySplit ks = key_split_exact(wgs, a.pos0 + a.tokens);
     if (ks.parts > 1) {
-        c.optional = true;
         const int st = launch_split<HW, OF32, false>(c, prefill_split_kernel<KV, HW, QS, PS, OF32>,
-                                                     "prefill_split_kernel", a, wgs, ks.parts, true,
+                                                     "prefill_split_kernel", a, wgs, ks.parts, 1, true,
                                                      2 * kThreads);
         if (st != 1) return st;
     }
@@ -2096,15 +2109,16 @@ int launch_f16(PfCtx& c, const PrefillArgs& a, bool* gated = nullptr) {
         PrefillArgs b = a;
         b.pair = c.pair && wgs >= 2 * 256;
         // one workgroup per CU
-        KeySplit ks = key_split_f16(wgs, a.pos0 + a.tokens);
+        KeySplit ks = key_split_f16(wgs, a.pos0 + a.tokens, GATED ? kStagedParts : kF16Parts);
         if (variant) ks = KeySplit{c.parts, c.parts > kMaxInKernelParts};
         ks.parts = clamp_parts(ks.parts, wgs);
         if (ks.parts > 1) {
+            const int must = required_parts(wgs, a.pos0 + a.tokens, 256);
             const int st = ks.two_step
                 ? launch_split<HW, false, GATED>(c, prefill_f16_kernel<HW, PS>, "prefill_f16_kernel",
-                                                 b, wgs, ks.parts, true, 2 * kThreads)
+                                                 b, wgs, ks.parts, must, true, 2 * kThreads)
                 : launch_split<HW, false, GATED>(c, prefill_f16_kernel<HW, PS, GATED>,
-                                                 "prefill_f16_kernel", b, wgs, ks.parts, false,
+                                                 "prefill_f16_kernel", b, wgs, ks.parts, must, false,
                                                  2 * kThreads);
             if (st != 1) return st;
         }
@@ -2140,7 +2154,9 @@ int launch_q8_kernel4(PfCtx& c, const PrefillArgs& a, bool* gated) {
             b.gate = a.taint;
         }
         const int st = launch_split<HW, false, true>(c, prefill_q8_kernel4<HW>, "prefill_q8_kernel4",
-                                                     b, wgs, ks.parts, ks.two_step, kThreads);
+                                                     b, wgs, ks.parts,
+                                                     required_parts(wgs, a.pos0 + a.tokens, 512),
+                                                     ks.two_step, kThreads);
         if (st != 1) {
             *gated = ks.two_step;
             return st;
@@ -2160,7 +2176,7 @@ template <int HW>
 int launch_q8_via_f16(PfCtx& c, const PrefillArgs& a, bool* gated) {
     const long long rows = (long long)((a.pos0 + a.tokens + 63) / 64 * 64) * a.hkv;
     const size_t bytes = (size_t)rows * kDim * 2;
-    void* ws = c.take(2 * bytes);
+    void* ws = c.take(2 * bytes, 2 * bytes);
     if (!ws) return launch_q8_kernel4<HW>(c, a, gated);
     uint16_t* kd = static_cast<uint16_t*>(ws);
     uint16_t* vd = kd + rows * kDim;
@@ -2283,8 +2299,9 @@ size_t prefill_workspace_len(int tokens, int hq, int hkv, int pos0, int kv, int 
     return c.need;
 }
 
-// caller_ws: the caller's workspace of ws_len bytes, at least prefill_workspace_len(); otherwise
-// the reference-signature call (the fixed workspace when this stream owns it).
+// caller_ws: the caller's workspace of ws_len bytes, at least the `required` of
+// prefill_workspace_len() (what it has no room for is left out); otherwise the reference-signature
+// call (the fixed workspace when this stream owns it).
 int prefill_launch(const float* q, const void* k, const void* v, void* o, int tokens, int hq,
                    int hkv, int pos0, int kv, int precision, bool caller_ws, void* ws,
                    size_t ws_len, hipStream_t stream, const int* layout) {

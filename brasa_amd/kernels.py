@@ -234,7 +234,8 @@ class Kernels:
 
     @staticmethod
     def flash_attention_workspace_len(shape: AttnShape, precision: PrefillPrecision) -> int:
-        """Bytes of caller workspace ``flash_attention_ws`` needs (no reference counterpart)."""
+        """Bytes of caller workspace for the full plan of ``flash_attention_ws``, which accepts
+        less where only a faster key split is left out (no reference counterpart)."""
         return int(lib().brasa_flash_attention_workspace_len(shape.c(), int(precision)))
 
     def flash_attention_ws(self, q, k, v, o, shape: AttnShape, precision: PrefillPrecision,

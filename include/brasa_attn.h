@@ -232,19 +232,24 @@ int brasa_flash_attention(const float* q, const void* k, const void* v, void* o,
 
 /*
  * No counterpart in the reference (its flash_attention encodes onto buffers the caller owns and
- * needs no scratch; lib.rs:1169-1248). Bytes of workspace brasa_flash_attention_ws needs for
- * this shape and precision: the key split's partials and the q8_0 staging the call's plan uses
- * (0 when it uses neither, or for an invalid shape). BRASA_PREFILL_F32, BRASA_PREFILL_F16_PF32 on
- * f32 and q8_0 caches and BRASA_PREFILL_F16 on f32 caches also accept less (or none), and split
- * the keys over as many parts as fit.
+ * needs no scratch; lib.rs:1169-1248). Bytes of workspace for the full plan of
+ * brasa_flash_attention_ws at this shape and precision: the key split's partials and the q8_0
+ * staging (0 when the plan uses neither, or for an invalid shape). Less is accepted down to what
+ * the call needs to run at all, and the keys are then split over as many parts as fit:
+ *   - nothing for BRASA_PREFILL_F32, for BRASA_PREFILL_F16_PF32 on f32 and q8_0 caches, and for
+ *     BRASA_PREFILL_F16 on f32 caches;
+ *   - otherwise the staging of a q8_0 call that stages its rows, and the partials of up to 8 key
+ *     parts: doubled from one (which needs none) while the launch fills at most half of the GPU
+ *     and every part keeps 1024 keys.
  */
 size_t brasa_flash_attention_workspace_len(brasa_attn_shape shape, int precision);
 
 /*
- * brasa_flash_attention_with on a caller-owned device workspace of workspace_len bytes (at least
- * brasa_flash_attention_workspace_len; BRASA_ERR_SCRATCH otherwise), for callers on any stream
- * that want the full plan. Allocates nothing. The same kernels and plan as the fixed-workspace
- * call, so the results are bit-identical to it. Calls in flight at the same time need distinct
+ * brasa_flash_attention_with on a caller-owned device workspace of workspace_len bytes, for callers
+ * on any stream that want the full plan. With brasa_flash_attention_workspace_len bytes: the same
+ * kernels and plan as the fixed-workspace call, so the results are bit-identical to it. With less,
+ * as far as that function accepts it: fewer key parts, the same result up to the split's rounding;
+ * BRASA_ERR_SCRATCH below that. Allocates nothing. Calls in flight at the same time need distinct
  * workspaces.
  */
 int brasa_flash_attention_ws(const float* q, const void* k, const void* v, void* o,

@@ -8,7 +8,8 @@ import re
 import pytest
 
 import brasa_amd
-from brasa_amd import AttnShape, BrasaError, Kernels, KvType, decode_partials_len, gqa_supported
+from brasa_amd import (AttnShape, BrasaError, Kernels, KvType, PrefillPrecision, decode_partials_len,
+                       gqa_supported)
 from brasa_amd._lib import SYMBOLS, lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -291,6 +292,56 @@ def test_prefill_workspace_len():
         16896 * 8 * 128 * 2 * 2 + 128 * 2 * 4 * 17 * 64 * 16
     assert wl(AttnShape(0, 32, 8, 128, 0, KvType.F16), F16) == 0
     assert wl(AttnShape(16, 32, 8, 64, 0, KvType.F16), F16) == 0  # invalid shape
+
+
+def _least_workspace(tokens, hq, hkv, pos0, kv, precision):
+    """What every flash_attention_ws call brings: the rows of a staged q8_0 call as f16, and the
+    partials of up to 8 key parts, doubled while half of the slots (one workgroup per CU, two for
+    q8_0 rows converted in registers) and parts of 16 64-key tiles allow."""
+    if precision != PrefillPrecision.F16 and kv != KvType.F16 or \
+            precision == PrefillPrecision.F32 or kv == KvType.F32:
+        return 0
+    group, lk = hq // hkv, pos0 + tokens
+    hw = 4 if group % 4 == 0 else 2 if group % 2 == 0 else 1
+    wgs = hq // hw * -(-tokens * hw // 128)
+    in_registers = kv == KvType.Q8_0 and tokens * lk < 384 * 384
+    parts = 1
+    while parts < 8 and wgs * parts * 2 <= (512 if in_registers else 256) and \
+            lk // (128 * parts) >= 16:
+        parts *= 2
+    staging = -(-lk // 64) * 64 * hkv * 512 if kv == KvType.Q8_0 and not in_registers else 0
+    return staging + (wgs * parts * 4 * 17 * 64 * 16 if parts > 1 else 0)
+
+
+def test_prefill_accepts_the_least_workspace():
+    """flash_attention_ws takes the least workspace of its shape, and the full one, over prompts,
+    chunks and short turns of every cache type, precision and GQA group, at odd lengths; an f16 call
+    refuses less than the smaller of the two. (Without a device a call that passes the check ends at
+    the device lookup.)"""
+    import random
+    from brasa_amd.device import device_count
+    if device_count():
+        pytest.skip("the pointers are not device memory")
+    r = random.Random(5)
+    k = Kernels()
+    for _ in range(3000):
+        hkv = r.choice([1, 2, 4, 8, 8, 8, 16, 32])
+        hq = hkv * r.choice([1, 2, 4, 4, 8])
+        tokens = int(2 ** r.uniform(0, 11.5))
+        pos0 = r.choice([0, int(2 ** r.uniform(0, 15))])
+        kv = r.choice([KvType.F32, KvType.F16, KvType.F16, KvType.Q8_0, KvType.Q8_0])
+        precision = r.choice(list(PrefillPrecision))
+        shape = AttnShape(tokens, hq, hkv, 128, pos0, kv)
+        need = Kernels.flash_attention_workspace_len(shape, precision)
+        least = _least_workspace(tokens, hq, hkv, pos0, kv, precision)
+
+        def code(size):
+            with pytest.raises(BrasaError) as e:
+                k.flash_attention_ws(256, 256, 256, 256, shape, precision, 256 if size else None, size)
+            return e.value.code
+        assert code(least) == code(need) == 4, (shape, precision, need, least)
+        if kv == KvType.F16 and min(least, need) > 0:
+            assert code(min(least, need) - 1) == 2, (shape, precision)
 
 
 def _plan(lens, hq=32, hkv=8, kv=KvType.F16):

@@ -567,6 +567,45 @@ def test_flash_nan_keys_of_whole_parts(kv, precision, tokens, pos0):
         assert np.array_equal(np.delete(o, 3, 1), np.delete(clean.reshape(o.shape), 3, 1))
 
 
+@pytest.mark.parametrize("kv,precision,tokens,pos0,least", [
+    (KvType.F16, "F16", 45, 1500, 0), (KvType.F16, "F16_PF32", 8, 800, 0),
+    (KvType.F16, "F16", 45, 7001, 4), (KvType.Q8_0, "F16", 5, 300, 0),
+    (KvType.Q8_0, "F16", 30, 9000, 8), (KvType.Q8_0, "F16", 45, 7001, 4)])
+def test_flash_smaller_workspace(kv, precision, tokens, pos0, least):
+    """F16 and F16_PF32 calls on less than the full workspace: `least` key parts of a query tile
+    (beside the staging of a staged q8_0 call) are enough, none at all where that is 0, and the keys
+    are split over what fits, at the bars. The whole workspace gives the fixed-workspace call's bits."""
+    prec = PrefillPrecision[precision]
+    synchronize()
+    assert lib().brasa_release_workspaces() == 0
+    k = Kernels()
+    rng = oracle.Rng(127 + tokens)
+    cap = (pos0 + tokens + 63) // 64 * 64
+    q = rng.vec(tokens * HQ * DIM, 2.0)
+    cache = KvPair(kv, rng.vec(cap * HKV * DIM, 2.0), rng.vec(cap * HKV * DIM, 3.0))
+    shape = AttnShape(tokens, HQ, HKV, DIM, pos0, kv)
+    need = Kernels.flash_attention_workspace_len(shape, prec)
+    unit = -(-tokens // 32) * HKV * PART_BYTES
+    staging = cap * HKV * DIM * 2 * 2 if kv == KvType.Q8_0 and tokens > 32 else 0
+    assert need > staging + max(least, 1) * unit
+    want = run_prefill(k, q, cache, tokens, HQ, HKV, pos0, prec)
+    ref16, vmax = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0, q16=True)
+    gq, ws = DeviceBuffer.from_array(q), DeviceBuffer(need)
+    for size in (need, staging + (least + 2) * unit + 1000, staging + least * unit):
+        ws.fill(0xFF)
+        o = DeviceBuffer(tokens * HQ * DIM * 2)
+        _say(f"prefill workspace {size} of {need} kv={kv.name_str} {precision} T={tokens}")
+        k.flash_attention_ws(gq, cache.kbuf, cache.vbuf, o, shape, prec, ws if size else None, size)
+        synchronize()
+        got = o.download(np.uint16).reshape(tokens, HQ, DIM)
+        if precision == "F16_PF32":
+            assert oracle.worst_f16(got, ref16, vmax) <= 1e-5, size
+        else:
+            a, r = bars(oracle.f16_to_f32(got), ref16)
+            assert a <= 2e-3 and r <= 1e-2, (size, a, r)
+        assert size < need or np.array_equal(got, want)
+
+
 Q8_RANGE_CASES = [(9, 2500, "k_large"), (40, 4000, "k_large"), (64, 500, "k_large"), (64, 500, "v_large"), (64, 500, "tiny"),
                   (384, 0, "k_large"), (384, 0, "v_large"), (384, 0, "tiny")]
 
