@@ -1824,7 +1824,10 @@ static int split_chunk(const int* lk, int n, long long total, int lk_max, int mo
 //    1024 to 16384 keys, 75K in all, took 72 us with 276 workgroups and takes 50 with 256). Where
 //    that leaves a batch of many sequences and heads (fewer than four splits each) with splits of
 //    more than kLongSplit keys, it takes two or four rounds of shorter ones instead, which balance
-//    better (32 KV heads, the same batch: 177 against 187 us; 8 KV heads: 53 against 50).
+//    better (32 KV heads, the same batch: 177 against 187 us; 8 KV heads: 53 against 50). One
+//    sequence's splits are of one length, with nothing to balance (64 to 512 KV heads, 2500 and
+//    16384 keys: four rounds 0.95 to 1.05 of the time of one), and one round of them fits the
+//    no-allocation entry point's array.
 //  * HPW: workgroups that read several adjacent KV heads load the HBM channels evenly (with one
 //    KV head per workgroup, the heads whose rows sit on the slower channels arrive ~2 us late at
 //    16K keys), but each merge group then has HPW * G query heads. The plan takes the largest HPW
@@ -1846,7 +1849,7 @@ DecodePlan decode_plan(const int* lk, int n, int ngroups, int G, int kv) {
         int chunk = 0;
         for (int wgs = kTargetWgs; wgs <= 4 * kTargetWgs; wgs *= 2) {
             chunk = split_chunk(lk, n, total, lk_max, std::max(wgs / rows, 1));
-            if (chunk <= kLongSplit || n * rows < kTargetWgs / 4) break;
+            if (n == 1 || chunk <= kLongSplit || n * rows < kTargetWgs / 4) break;
         }
         const int splits = (int)(((long long)lk_max + chunk - 1) / chunk);
         if (hpw > 1) {

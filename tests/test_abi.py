@@ -388,6 +388,21 @@ def test_decode_plan_fills_the_gpu_once(hq, hkv, kv):
         assert least == 256 or n * rows >= 64
 
 
+@pytest.mark.parametrize("kv", [KvType.F16, KvType.Q8_0, KvType.F32])
+def test_decode_noalloc_holds_every_shape(kv):
+    """A single sequence's plan stays within one workgroup per CU (one split where the head groups
+    alone exceed that), so the partials of any head count and length fit the array of
+    brasa_decode_attention_lanes_noalloc."""
+    for hkv in [*range(1, 65), 96, 128, 192, 256, 320, 512, 768, 1024]:
+        for group in (1, 2, 4, 8):
+            if hkv * group > 1024:
+                continue
+            for lk in (1, 300, 2500, 9000, 16384, 131072, 1 << 24, 1 << 30):
+                _, hpw, (splits,) = _plan([lk], hkv * group, hkv, kv)
+                assert splits == 1 or splits * -(-hkv // hpw) <= 256, (hkv, group, lk)
+                assert hkv * group * splits * 130 <= 1 << 20, (hkv, group, lk)
+
+
 @pytest.mark.parametrize("lens,hq,hkv,kv", [
     ([1], 32, 8, KvType.F16), ([37], 32, 8, KvType.Q8_0), ([128], 32, 8, KvType.F16),
     ([129], 32, 8, KvType.F16), ([2048], 32, 8, KvType.F16), ([4096], 32, 8, KvType.Q8_0),
