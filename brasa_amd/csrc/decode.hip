@@ -55,10 +55,12 @@ constexpr int kWavesF32 = 8;
 // covers with 8 waves (kWavesF16 / kWavesQ8).
 constexpr int kMaxMergeHeads = 16;
 // Merge size bounds of the plan, in (query heads x splits) of a merge group; the last workgroup
-// loads 520 bytes per (query head, split). Up to kMergeWorkSmall (106 KB) for any layout; up to
+// loads 520 bytes per (query head, split). Up to kMergeWorkSmall (66 KB) for any layout; up to
 // kMergeWorkLong (~200 KB) when splits are long (>= kLongChunk keys), where streaming several KV
-// heads per workgroup gains more than the larger merge costs.
-constexpr int kMergeWorkSmall = 208;
+// heads per workgroup gains more than the larger merge costs. With a bound of 208, f16 and two
+// heads per workgroup: 16 heads over 8 at 6100 keys 11.2 us, 10.0 with this one and one head
+// (8300: 12.4, 11.5); 64 over 16 at 3000 11.2, 9.8; sixteen batches of 3 to 8 sequences 0.98 to 1.06.
+constexpr int kMergeWorkSmall = 128;
 constexpr int kMergeWorkLong = 384;
 constexpr int kLongChunk = 512;
 constexpr int kLongSplit = 1024;  // keys per split above which a large batch takes more rounds
