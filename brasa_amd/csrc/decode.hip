@@ -1731,7 +1731,7 @@ int launch(const DecodeArgs<NS>& a, int hpw, int cols, hipStream_t stream) {
     if (hpw == 1) return launch_hpw<KV, G, NS, 1>(a, cols, stream);
     if constexpr (2 * G <= kMaxMergeHeads)
         if (hpw == 2) return launch_hpw<KV, G, NS, 2>(a, cols, stream);
-    if constexpr (4 * G <= kMaxMergeHeads)
+    if constexpr (4 * G <= kMaxMergeHeads && KV != BRASA_KV_F32)  // (f32 plans take two at most)
         if (hpw == 4) return launch_hpw<KV, G, NS, 4>(a, cols, stream);
     return set_error(BRASA_ERR_UNSUPPORTED, "decode: %d head groups per workgroup not compiled", hpw);
 }
