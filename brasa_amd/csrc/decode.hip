@@ -55,12 +55,13 @@ constexpr int kWavesF32 = 8;
 // covers with 8 waves (kWavesF16 / kWavesQ8).
 constexpr int kMaxMergeHeads = 16;
 // Merge size bounds of the plan, in (query heads x splits) of a merge group; the last workgroup
-// loads 520 bytes per (query head, split). Up to kMergeWorkSmall (66 KB) for any layout; up to
+// loads 520 bytes per (query head, split). Up to kMergeWorkSmall (81 KB) for any layout; up to
 // kMergeWorkLong (~200 KB) when splits are long (>= kLongChunk keys), where streaming several KV
-// heads per workgroup gains more than the larger merge costs. With a bound of 208, f16 and two
-// heads per workgroup: 16 heads over 8 at 6100 keys 11.2 us, 10.0 with this one and one head
-// (8300: 12.4, 11.5); 64 over 16 at 3000 11.2, 9.8; sixteen batches of 3 to 8 sequences 0.98 to 1.06.
-constexpr int kMergeWorkSmall = 128;
+// heads per workgroup gains more than the larger merge costs. f16, two heads per workgroup and 192
+// pairs against one head: 16 heads over 8 at 6100 keys 11.2 us, 10.0 (208 pairs, 8300 keys: 12.4,
+// 11.5); 64 over 16 at 3000 keys 11.2, 9.8. Batches of 2 to 12 sequences: 176 to 200 pairs 0.98 to
+// 1.06 of the time of half the heads, 132 to 160 pairs 0.97 to 1.04 (groups of 8: 1.07 to 1.10).
+constexpr int kMergeWorkSmall = 160;
 constexpr int kMergeWorkLong = 384;
 constexpr int kLongChunk = 512;
 constexpr int kLongSplit = 1024;  // keys per split above which a large batch takes more rounds
@@ -1822,8 +1823,8 @@ static int split_chunk(const int* lk, int n, long long total, int lk_max, int mo
 // launch. A function of the lengths and head counts only, so a call's result never depends on
 // anything else.
 //  * Split length: the shortest that keeps the launch within one workgroup per CU (a workgroup
-//    fills its CU, so one workgroup more would run after the others: a batch of 8 sequences of
-//    1024 to 16384 keys, 75K in all, took 72 us with 276 workgroups and takes 50 with 256). Where
+//    fills its CU, so one workgroup more would run after the others: 8 sequences of 4922,
+//    10733, 9940, 3160, 7085, 16030, 10918 and 8790 keys: 71.6 us with 268 workgroups, 50.5 with 252). Where
 //    that leaves a batch of many sequences and heads (fewer than four splits each) with splits of
 //    more than kLongSplit keys, it takes two or four rounds of shorter ones instead, which balance
 //    better (32 KV heads, the same batch: 177 against 187 us; 8 KV heads: 53 against 50). One

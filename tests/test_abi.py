@@ -390,7 +390,7 @@ def test_decode_plan_fills_the_gpu_once(hq, hkv, kv):
 
 @pytest.mark.parametrize("hq,hkv", [(32, 8), (16, 8), (64, 16), (32, 4), (32, 32), (20, 5)])
 def test_decode_plan_bounds_the_merge(hq, hkv):
-    """Several head groups share a workgroup only where the last one to arrive merges at most 128
+    """Several head groups share a workgroup only where the last one to arrive merges at most 160
     (query head, split) pairs, or 384 where the splits are 512 keys or longer."""
     import random
     r = random.Random(hq + hkv)
@@ -399,7 +399,7 @@ def test_decode_plan_bounds_the_merge(hq, hkv):
         for kv in KvType:
             chunk, hpw, splits = _plan(lens, hq, hkv, kv)
             pairs = hq // hkv * hpw * max(splits)
-            assert hpw == 1 or pairs <= (384 if chunk >= 512 else 128), (lens, kv)
+            assert hpw == 1 or pairs <= (384 if chunk >= 512 else 160), (lens, kv)
 
 
 @pytest.mark.parametrize("kv", [KvType.F16, KvType.Q8_0, KvType.F32])
