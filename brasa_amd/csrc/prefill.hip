@@ -1958,15 +1958,22 @@ KeySplit split_in_kernel(long long wgs, int tiles, int slots) {
 }
 constexpr int kFewTiles = 16;  // query tiles up to which the merge is a launch of its own
 int key_tiles(int keys) { return (keys + kTile - 1) / kTile; }
-// the two-group f16 kernel, one workgroup per CU; `most` parts
-KeySplit key_split_f16(long long wgs, int keys, int most) {
+// The two-group f16 kernel, one workgroup per CU. `staged`: a launch a q8_0 call takes on staged
+// rows too (several query tiles). Where 8 parts are required it takes those or 16, nothing between:
+// a workspace of the staging and 8 parts is then the whole one from 8192 keys on, up to where twice
+// the parts are worth a larger one (64 tokens after 8192: 28.1 us with 8, 26.1 with 13; q8_0 40.5 and
+// 38.1; 60 after 16000 39.3 with 8, 33.6 with 16).
+KeySplit key_split_f16(long long wgs, int keys, bool staged, int required) {
     const int tiles = key_tiles(keys);
     if (tiles < 12) return KeySplit{1, false};
-    if (wgs <= kFewTiles) return split_two_step(4.5, wgs, tiles, 256, most);
+    if (wgs <= kFewTiles) {
+        const KeySplit k = split_two_step(4.5, wgs, tiles, 256, 16);
+        return staged && required == 8 && k.parts < 16 ? KeySplit{8, true} : k;
+    }
     const KeySplit k = split_in_kernel(wgs, tiles, 256);
     // more than 6 parts: the own launch once the keys are long enough to pay for it
     if (k.parts <= 6) return k;
-    return tiles >= 64 ? KeySplit{(int)std::min<long long>(256 / wgs, most), true} : KeySplit{6, false};
+    return tiles >= 64 ? KeySplit{(int)(256 / wgs), true} : KeySplit{6, false};
 }
 // prefill_q8_kernel4, two workgroups per CU. The merge launch also reads the range flag, in
 // place of the launch of prefill_exact_kernel an unsplit call needs, so it pays from few tiles on
@@ -1985,12 +1992,6 @@ KeySplit key_split_exact(long long wgs, int keys) {
     if (tiles < (wgs <= kFewTiles ? 4 : wgs <= 64 ? 6 : 12)) return KeySplit{1, false};
     return split_two_step(9.0, wgs, tiles, 256, std::min(tiles, kMaxKeyParts));
 }
-
-// f16 rows staged from a q8_0 cache: no more parts than required_parts can ask for, so that a
-// workspace that holds the staging and 8 parts is the whole one (64 tokens after 8192, which ask
-// for 8: 41.0 us; 13 parts, as the f16 rule has it, 38.1; 45 after 7001 36.1 and 34.6 with 12)
-constexpr int kStagedParts = 8;
-constexpr int kF16Parts = 16;
 
 // parts within the limits of the workspace layout and the counter slot, else 1
 int clamp_parts(int parts, long long wgs) {
@@ -2109,11 +2110,11 @@ int launch_f16(PfCtx& c, const PrefillArgs& a, bool* gated = nullptr) {
         PrefillArgs b = a;
         b.pair = c.pair && wgs >= 2 * 256;
         // one workgroup per CU
-        KeySplit ks = key_split_f16(wgs, a.pos0 + a.tokens, GATED ? kStagedParts : kF16Parts);
+        const int must = required_parts(wgs, a.pos0 + a.tokens, 256);
+        KeySplit ks = key_split_f16(wgs, a.pos0 + a.tokens, a.ntiles > 1, must);
         if (variant) ks = KeySplit{c.parts, c.parts > kMaxInKernelParts};
         ks.parts = clamp_parts(ks.parts, wgs);
         if (ks.parts > 1) {
-            const int must = required_parts(wgs, a.pos0 + a.tokens, 256);
             const int st = ks.two_step
                 ? launch_split<HW, false, GATED>(c, prefill_f16_kernel<HW, PS>, "prefill_f16_kernel",
                                                  b, wgs, ks.parts, must, true, 2 * kThreads)
