@@ -62,6 +62,7 @@ def test_batch_mixed_short_and_many_sequences():
 
 @pytest.mark.parametrize("group", [1, 2, 8])
 def test_batch_other_groups(group):
+    """A small batch of the other GQA groups, one head group to a workgroup."""
     hkv = 4
     hq = hkv * group
     lens = [700, 33, 2500]
@@ -73,7 +74,9 @@ def test_batch_other_groups(group):
 
 
 @pytest.mark.parametrize("kv,group", [(KvType.F32, 4), (KvType.F32, 8), (KvType.F16, 4),
-                                      (KvType.F16, 8), (KvType.Q8_0, 4), (KvType.Q8_0, 2)])
+                                      (KvType.F16, 8), (KvType.Q8_0, 4), (KvType.Q8_0, 2),
+                                      (KvType.F32, 1), (KvType.F32, 2), (KvType.F16, 1),
+                                      (KvType.F16, 2), (KvType.Q8_0, 1), (KvType.Q8_0, 8)])
 def test_batch_several_heads_per_workgroup(kv, group):
     """Five KV heads, two or four to a workgroup: the last grid row holds one head group and
     places past it. Lengths around the edges of units, blocks and splits."""

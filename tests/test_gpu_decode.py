@@ -117,9 +117,8 @@ def test_decode_q_at_any_float(kv, hq):
 
 @pytest.mark.parametrize("kv", KVS)
 def test_decode_partial_head_group_row(kv):
-    # six KV heads at GQA group 4: at short lengths the plan puts four head groups in a
-    # workgroup, so the second grid row holds two real head groups and two past the last one
-    # (waves without keys, merge threads past hq)
+    # six KV heads at GQA group 4, a head count that is no power of two: the plan puts one head
+    # group in a workgroup at every length (test_decode_partial_row_of_several_groups has more)
     k = Kernels()
     rng = oracle.Rng(31)
     hq, hkv = 24, 6
@@ -133,6 +132,26 @@ def test_decode_partial_head_group_row(kv):
         want, vmax = oracle.attention(q, cache.k, cache.v, 1, hq, hkv, DIM, pos0)
         w = max(w, oracle.worst(got, want, vmax))
     assert w <= 1e-5, w
+
+
+@pytest.mark.parametrize("kv,group,hkv,lk,hpw", [
+    (KvType.F16, 1, 30, 4000, 4), (KvType.F16, 2, 30, 16400, 4), (KvType.F16, 4, 31, 2100, 2),
+    (KvType.Q8_0, 1, 30, 4000, 4), (KvType.Q8_0, 4, 31, 2100, 2), (KvType.F32, 2, 31, 2100, 2),
+    (KvType.F32, 4, 31, 2100, 2)])
+def test_decode_partial_row_of_several_groups(kv, group, hkv, lk, hpw):
+    """Two or four head groups to a workgroup, and a last grid row with places past the last head
+    group (waves without keys, merge threads past hq)."""
+    from test_abi import _plan
+    hq = hkv * group
+    assert _plan([lk], hq, hkv, kv)[1] == hpw and hkv % hpw
+    k = Kernels()
+    rng = oracle.Rng(33)
+    q = rng.vec(hq * DIM, 2.0)
+    cache = KvPair(kv, rng.vec(lk * hkv * DIM, 2.0), rng.vec(lk * hkv * DIM, 3.0))
+    _say(f"decode lanes hq={hq} hkv={hkv} kv={kv.name_str} lk={lk} hpw={hpw}")
+    got = run_decode(k, "lanes", q, cache, hq, hkv, lk - 1)
+    want, vmax = oracle.attention(q, cache.k, cache.v, 1, hq, hkv, DIM, lk - 1)
+    assert oracle.worst(got, want, vmax) <= 1e-5
 
 
 def test_decode_non_power_of_two_group():

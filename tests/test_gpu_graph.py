@@ -122,7 +122,10 @@ def test_graph_decode_noalloc_and_batch():
 
 
 @pytest.mark.parametrize("kv,tokens,pos0", [(KvType.F16, 512, 0), (KvType.F16, 128, 8192),
-                                            (KvType.Q8_0, 64, 0), (KvType.Q8_0, 384, 0)])
+                                            (KvType.Q8_0, 64, 0), (KvType.Q8_0, 384, 0),
+                                            # the key split's merge as a launch of its own
+                                            (KvType.F16, 9, 7000), (KvType.Q8_0, 9, 2500),
+                                            (KvType.Q8_0, 45, 4000), (KvType.F32, 40, 3000)])
 def test_graph_prefill(kv, tokens, pos0):
     k = Kernels()
     rng = np.random.default_rng(7200 + tokens + pos0)

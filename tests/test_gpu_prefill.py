@@ -281,7 +281,8 @@ def test_flash_key_split(parts):
 
 def test_flash_key_split_q8():
     # q8_0 cache, F16 precision (the f16 kernels on the dequantised rows): 64 tokens after 8192
-    # cached positions is 16 workgroups, which the launch splits into 8 key parts by itself
+    # cached positions is 16 workgroups, which the launch splits into 8 key parts by itself,
+    # merged by a launch of their own
     k = Kernels()
     rng = oracle.Rng(89)
     tokens, pos0, hq, hkv = 64, 8192, HQ, HKV
@@ -300,8 +301,8 @@ def test_flash_key_split_q8():
 
 
 def test_flash_key_split_q8_kernel():
-    # a launch below the dequantisation threshold stays on the q8_0 kernel: 32 tokens after
-    # 4000 cached positions is 8 workgroups, split into 2 key parts by size
+    # a launch of one query tile stays on the q8_0 kernel: 32 tokens after 4000 cached positions
+    # is 8 workgroups, split into 21 key parts by size, merged by a launch of their own
     k = Kernels()
     rng = oracle.Rng(96)
     tokens, pos0 = 32, 4000
@@ -315,6 +316,30 @@ def test_flash_key_split_q8_kernel():
     ref16, vmax = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0, q16=True)
     a, r = bars(oracle.f16_to_f32(oh), ref16)
     print(f"q8_0 kernel key split: F16 max-abs {a:.2e} max-rel {r:.2e}")
+    assert a <= 2e-3 and r <= 1e-2, (a, r)
+
+
+@pytest.mark.parametrize("tokens,pos0,parts", [(70, 1500, 6), (150, 700, 3)])
+def test_flash_q8_kernel_in_launch_merge(tokens, pos0, parts):
+    """prefill_q8_kernel4's key split of more than 16 query tiles, merged by the last part to
+    arrive: the F16 bars, equal bits in repeat calls, and the workspace of `parts` parts."""
+    synchronize()
+    assert lib().brasa_release_workspaces() == 0
+    tiles = -(-tokens // 32) * HKV
+    assert tiles > 16 and Kernels.flash_attention_workspace_len(
+        AttnShape(tokens, HQ, HKV, DIM, pos0, KvType.Q8_0), PrefillPrecision.F16) == \
+        tiles * parts * PART_BYTES
+    k = Kernels()
+    rng = oracle.Rng(131 + tokens)
+    cap = (pos0 + tokens + 63) // 64 * 64
+    q = rng.vec(tokens * HQ * DIM, 2.0)
+    cache = KvPair(KvType.Q8_0, rng.vec(cap * HKV * DIM, 2.0), rng.vec(cap * HKV * DIM, 3.0))
+    _say(f"prefill q8_0 kernel in-launch merge F16 T={tokens} pos0={pos0}")
+    oh = run_prefill(k, q, cache, tokens, HQ, HKV, pos0, PrefillPrecision.F16)
+    assert np.array_equal(oh, run_prefill(k, q, cache, tokens, HQ, HKV, pos0,
+                                          PrefillPrecision.F16))
+    ref16, _ = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0, q16=True)
+    a, r = bars(oracle.f16_to_f32(oh), ref16)
     assert a <= 2e-3 and r <= 1e-2, (a, r)
 
 
@@ -433,33 +458,45 @@ TWO_STEP = [(KvType.F16, "F16", 1, 767), (KvType.F16, "F16_PF32", 33, 1000),
             (KvType.Q8_0, "F16", 45, 4099), (KvType.F32, "F32", 2, 255),
             (KvType.F32, "F32", 7, 6200), (KvType.Q8_0, "F16_PF32", 64, 700),
             (KvType.F16, "F32", 100, 333)]
+# (hq, hkv, the same): GQA groups 1, 2 and 8 (the merge of one and two query heads per workgroup,
+# and two workgroups of four a KV head), more than 16 query tiles, and, at pos0 0, parts without
+# a key of the first query tiles
+TWO_STEP_HEADS = [(8, 8, KvType.F16, "F16", 100, 1500), (8, 8, KvType.Q8_0, "F16", 9, 1200),
+                  (8, 8, KvType.Q8_0, "F16", 129, 2500), (8, 8, KvType.F32, "F32", 130, 800),
+                  (16, 8, KvType.F16, "F16_PF32", 65, 1100), (16, 8, KvType.Q8_0, "F16", 20, 900),
+                  (16, 8, KvType.F32, "F16", 33, 1700), (64, 8, KvType.F16, "F16", 31, 2100),
+                  (64, 8, KvType.Q8_0, "F16_PF32", 12, 600), (HQ, HKV, KvType.F16, "F16", 70, 4100),
+                  (4, 1, KvType.F32, "F32", 383, 0), (4, 1, KvType.Q8_0, "F16_PF32", 300, 0),
+                  (4, 1, KvType.Q8_0, "F16", 383, 0)]
 
 
-@pytest.mark.parametrize("kv,precision,tokens,pos0", TWO_STEP)
-def test_flash_key_split_own_launch(kv, precision, tokens, pos0):
+@pytest.mark.parametrize("hq,hkv,kv,precision,tokens,pos0",
+                         [(HQ, HKV, *c) for c in TWO_STEP] + TWO_STEP_HEADS)
+def test_flash_key_split_own_launch(hq, hkv, kv, precision, tokens, pos0):
     """Key splits merged by prefill_merge_kernel, at the bars of the unsplit kernels; repeat calls
     give equal bits (the parts merge in a fixed order), and garbage past the last key is masked."""
     prec = PrefillPrecision[precision]
     synchronize()
     assert lib().brasa_release_workspaces() == 0
     assert Kernels.flash_attention_workspace_len(
-        AttnShape(tokens, HQ, HKV, DIM, pos0, kv), prec) > 0
+        AttnShape(tokens, hq, hkv, DIM, pos0, kv), prec) > 0
     k = Kernels()
     rng = oracle.Rng(103 + tokens)
     lk = pos0 + tokens
     cap = (lk + 63) // 64 * 64
-    q = rng.vec(tokens * HQ * DIM, 2.0)
-    kk, vv = rng.vec(cap * HKV * DIM, 2.0), rng.vec(cap * HKV * DIM, 3.0)
-    kk[lk * HKV * DIM:], vv[lk * HKV * DIM:] = 3e4, -3e4
+    q = rng.vec(tokens * hq * DIM, 2.0)
+    kk, vv = rng.vec(cap * hkv * DIM, 2.0), rng.vec(cap * hkv * DIM, 3.0)
+    kk[lk * hkv * DIM:], vv[lk * hkv * DIM:] = 3e4, -3e4
     cache = KvPair(kv, kk, vv)
-    _say(f"prefill own-launch merge kv={kv.name_str} {precision} T={tokens} pos0={pos0}")
-    o = run_prefill(k, q, cache, tokens, HQ, HKV, pos0, prec)
-    assert np.array_equal(o, run_prefill(k, q, cache, tokens, HQ, HKV, pos0, prec))
+    _say(f"prefill own-launch merge hq={hq} hkv={hkv} kv={kv.name_str} {precision} T={tokens} "
+         f"pos0={pos0}")
+    o = run_prefill(k, q, cache, tokens, hq, hkv, pos0, prec)
+    assert np.array_equal(o, run_prefill(k, q, cache, tokens, hq, hkv, pos0, prec))
     if precision == "F32":
-        raw, vmax = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0)
+        raw, vmax = oracle.attention(q, cache.k, cache.v, tokens, hq, hkv, DIM, pos0)
         assert oracle.worst(o, raw, vmax) <= 1e-5
         return
-    ref16, vmax = oracle.attention(q, cache.k, cache.v, tokens, HQ, HKV, DIM, pos0, q16=True)
+    ref16, vmax = oracle.attention(q, cache.k, cache.v, tokens, hq, hkv, DIM, pos0, q16=True)
     if precision == "F16_PF32":
         assert oracle.worst_f16(o, ref16, vmax) <= 1e-5
     else:
@@ -606,7 +643,7 @@ def test_flash_smaller_workspace(kv, precision, tokens, pos0, least):
         assert size < need or np.array_equal(got, want)
 
 
-Q8_RANGE_CASES = [(9, 2500, "k_large"), (40, 4000, "k_large"), (64, 500, "k_large"), (64, 500, "v_large"), (64, 500, "tiny"),
+Q8_RANGE_CASES = [(9, 2500, "k_large"), (40, 4000, "k_large"), (70, 1500, "k_large"), (64, 500, "k_large"), (64, 500, "v_large"), (64, 500, "tiny"),
                   (384, 0, "k_large"), (384, 0, "v_large"), (384, 0, "tiny")]
 
 
@@ -656,8 +693,8 @@ def test_flash_q8_scales_outside_f16(tokens, pos0, kind):
 
 
 def test_flash_key_split_chosen_by_size():
-    # 128 query tiles x 8 head groups is below half the CUs: the launch splits the keys by
-    # itself (two parts at 64 tokens after 8192 cached positions)
+    # 16 workgroups (two query tiles a KV head) leave most CUs idle: the launch splits the keys by
+    # itself (8 parts at 64 tokens after 8192 cached positions, merged by a launch of their own)
     k = Kernels()
     rng = oracle.Rng(83)
     tokens, pos0, hq, hkv = 64, 8192, HQ, HKV
