@@ -336,14 +336,17 @@ def profile_run(k: Kernels, stream: Stream, what: str) -> int:
     src.free()
     dst.free()
     decode_cases = {"decode": (16384, KvType.F16), "decode_q8": (16384, KvType.Q8_0),
-                    "decode_4k": (4096, KvType.F16), "decode_32k": (32768, KvType.F16)}
+                    "decode_4k": (4096, KvType.F16), "decode_32k": (32768, KvType.F16),
+                    "decode_f32": (2048, KvType.F32)}
     f16, q8, pf32 = KvType.F16, KvType.Q8_0, PrefillPrecision.F16_PF32
     prefill_cases = {"prefill": (2048, 0, f16, PrefillPrecision.F16),
                      "prefill_8k": (8192, 0, f16, PrefillPrecision.F16),
                      "prefill_chunk": (512, 16384, f16, PrefillPrecision.F16),
                      "prefill_pf32": (2048, 0, f16, pf32),
                      "prefill_q8": (2048, 0, q8, PrefillPrecision.F16),
-                     "prefill_q8_chunk": (512, 16384, q8, PrefillPrecision.F16)}
+                     "prefill_q8_chunk": (512, 16384, q8, PrefillPrecision.F16),
+                     "prefill_turn": (45, 7001, f16, PrefillPrecision.F16),
+                     "prefill_f32": (1000, 0, KvType.F32, PrefillPrecision.F32)}
     if what in decode_cases:
         lk, kv = decode_cases[what]
         layers = DecodeLayers(k, lk, kv, stream)
@@ -370,7 +373,8 @@ def main() -> int:
     ap.add_argument("--profile", choices=("decode", "decode_q8", "decode_4k", "decode_32k",
                                           "decode_ragged", "prefill", "prefill_8k",
                                           "prefill_chunk", "prefill_pf32", "prefill_q8",
-                                          "prefill_q8_chunk"),
+                                          "prefill_q8_chunk", "decode_f32", "prefill_turn",
+                                          "prefill_f32"),
                     help="short fixed run for rocprofv3 (kernel trace / counters), no JSON line")
     args = ap.parse_args()
     if args.gpus != 1:

@@ -134,7 +134,7 @@ def report(r: dict) -> str:
 def main() -> None:
     ap = argparse.ArgumentParser(description=__doc__.split("\n\n")[0])
     ap.add_argument("--lk", type=int, default=16384)
-    ap.add_argument("--kv", default="f16", choices=["f16", "q8_0"])
+    ap.add_argument("--kv", default="f16", choices=["f16", "q8_0", "f32"])
     ap.add_argument("--reps", type=int, default=5)
     a = ap.parse_args()
     print(report(run(a.lk, a.kv, a.reps)), flush=True)
