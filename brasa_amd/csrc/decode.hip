@@ -22,13 +22,13 @@
 //     of its head group; the last workgroup to arrive merges all the splits and writes o. One
 //     kernel per call: a second dependent launch for the merge costs ~3 us per layer here;
 //   * q8_0: codes are exact in f16; K scales multiply the per-32-dim-group MFMA partials (one
-//     MFMA k-step is one group), V scales are folded into P per group; f32 caches are split
-//     hi + lo like Q.
-// A single-sequence call's result is a function of (q, k, v, lk) only: the split length and the
-// wave count per workgroup depend on lk alone (no tuning knob changes them) and every merge runs
-// in a fixed order. A batched launch shares one split length, taken from the batch's total keys,
-// so a sequence's splits, and with them the last bits of its result, can differ from the
-// single-sequence call (both within the decode tolerance).
+//     MFMA k-step is one group), V scales are folded into P per group; f32 caches stay f32, on
+//     the f32 matrix instructions.
+// A single-sequence call's result is a function of (q, k, v, lk) only: the launch plan depends on lk,
+// the head counts and the cache type (no tuning knob changes it) and every merge runs in a fixed
+// order. A batched launch shares one split length, taken from all its lengths, so a sequence's
+// splits, and with them the last bits of its result, can differ from the single-sequence call
+// (both within the decode tolerance).
 #include <atomic>
 #include <cstring>
 #include <mutex>
@@ -124,7 +124,7 @@ struct SeqDesc {
     const uint8_t* v;
     size_t part_off;      // floats: this sequence's partials (acc [hq][splits][128], then ml)
     int lk;               // keys
-    int chunk;            // keys per split (a function of lk alone)
+    int chunk;            // keys per split (DecodePlan; one for the whole launch)
     int splits;
     int split0;           // first grid column of this sequence
 };
@@ -826,10 +826,10 @@ decode_f16_kernel(DecodeArgs<NS> a) {
 // MFMA does 4 heads x 4 keys (or dims) in each block with no conversion, where f16 matrix
 // instructions would need every value split into hi + lo halves (the former kernel spent ~1,000
 // instructions of a 32-key block on those splits and on a transposed V tile in LDS).
-// Workgroup = one head group x one split, W wave64; a wave walks units of 16 keys (half a 32-key
-// block, so a 128-key split still feeds 8 waves), w, w + W, ... A unit is 16 loads of 16 bytes per
-// lane, K and V straight into registers, each instruction covering 4 whole rows; a wave keeps
-// two units in flight, with exact waits (one: the same within 1 %, 4097 keys 11.35 -> 11.6 us).
+// Workgroup = HPW (1 or 2) adjacent head groups x one split, W wave64; a wave walks units of 16 keys
+// (half a 32-key block, so a 128-key split still feeds 8 waves), ks, ks + KS, ... A unit is 16 loads
+// of 16 bytes per lane, K and V straight into registers, two instructions covering 4 whole rows; a
+// wave keeps two units in flight, with exact waits (one: 0 to 2 % slower, 4097 keys 11.35 -> 11.6 us).
 // Lane l = 16 u + c = 4 b + j.
 //  * S: block b takes dims 8 b .. 8 b + 7, A = q of head j (4 lanes: 4 heads), B = K of key
 //    4 t + j: D of lane (b, j) is the partial score of key 4 t + j for the 4 heads. The 16 blocks
@@ -1827,7 +1827,8 @@ static int split_chunk(const int* lk, int n, long long total, int lk_max, int mo
 //    10733, 9940, 3160, 7085, 16030, 10918 and 8790 keys: 71.6 us with 268 workgroups, 50.5 with 252). Where
 //    that leaves a batch of many sequences and heads (fewer than four splits each) with splits of
 //    more than kLongSplit keys, it takes two or four rounds of shorter ones instead, which balance
-//    better (32 KV heads, the same batch: 177 against 187 us; 8 KV heads: 53 against 50). One
+//    better (32 KV heads: these 8 sequences 180 against 184 us, 16 of 512 to 8192 keys f16 144
+//    against 162, f32 295 against 442; with 8 KV heads the 8 take 53 against 50). One
 //    sequence's splits are of one length, with nothing to balance (64 to 512 KV heads, 2500 and
 //    16384 keys: four rounds 0.95 to 1.05 of the time of one), and one round of them fits the
 //    no-allocation entry point's array.

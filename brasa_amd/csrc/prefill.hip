@@ -347,9 +347,10 @@ __device__ __forceinline__ void q_convert_half(const u32x4 (&raw)[8], float scal
 //
 // Each 64-key stage is copied HBM -> LDS by global_load_lds_dwordx4 (raw f16 rows, 16-byte chunks
 // XOR-swizzled so the operand reads are bank-conflict free), K A-operands are ds_read_b128 of
-// those rows and V^T A-operands are ds_read_tr16_b64 of the same row-major tile. Two stages alternate so stage i + 1 streams in while stage i is contracted. The O
-// accumulator is only rescaled when a column's running max grows by more than 2^8 (P then stays
-// below 256, well inside f16), and masking runs only on tiles that cross the diagonal.
+// those rows and V^T A-operands are ds_read_tr16_b64 of the same row-major tile. Two stages
+// alternate so stage i + 1 streams in while stage i is contracted. The O accumulator is only
+// rescaled when a column's running max grows by more than 2^8 (P then stays below 256, well inside
+// f16), and masking runs only on tiles that cross the diagonal.
 constexpr int kStageHalves = kTile * kDim;  // one 64 x 128 f16 tile
 
 // physical 16-byte chunk of logical chunk c in row r
@@ -383,11 +384,12 @@ __device__ __forceinline__ void store_key_part(const PrefillArgs& a, int tile, i
 
 // Key split merged in the kernel (up to kMaxInKernelParts parts): after its two key groups have
 // merged, each group-0 wave of part `part` holds (acc, m, lsum) of its 32 queries over that
-// part's keys. It stores them to a.part (part_state) with device-coherent stores, waits until they are visible and counts its arrival
-// on the wave's counter (atomic inc wrapping at kparts - 1, so the last arrival returns it to
-// zero). The last wave to arrive loads every part's state and merges them in part order (max
-// first, then 2^(m_p - max)-weighted sums), so the result does not depend on the arrival
-// order; it returns true and its acc / lsum then hold the merged state. Other waves return false.
+// part's keys. It stores them to a.part (part_state) with device-coherent stores, waits until they
+// are visible and counts its arrival on the wave's counter (atomic inc wrapping at kparts - 1, so
+// the last arrival returns it to zero). The last wave to arrive loads every part's state and merges
+// them in part order (max first, then 2^(m_p - max)-weighted sums), so the result does not depend on
+// the arrival order; it returns true and its acc / lsum then hold the merged state. Other waves
+// return false.
 __device__ __forceinline__ bool merge_key_parts(const PrefillArgs& a, int tile, int part, int qw,
                                              int lane, f32x16 (&acc)[4], float& m_used,
                                              float& lsum) {
@@ -1061,7 +1063,7 @@ prefill_f16_kernel4(PrefillArgs a) {
 // every value to f16(code * scale) (the exact dequantised value rounded once, like Q * scale in
 // this precision; codes4_to_f16 gives the codes exactly, one packed f16 multiply the rounding)
 // and writes the f16 rows in the swizzled layouts the f16 kernels read, so the contraction runs
-// at one MFMA per product instead of the generic kernel's hi / lo splits.
+// at one MFMA per product instead of prefill_split_kernel's hi / lo splits.
 struct Q8Rows {
     u32x4 kc[2], vc[2];   // 16 codes of rows r0, r0 + 8 (lane's 16-byte chunk)
     uint32_t ks[2], vs[2];  // the f16 scale of the chunk's 32-group, per row (low half)
@@ -1772,8 +1774,8 @@ prefill_split_kernel(PrefillArgs a) {
 // The merge of a key split as a launch of its own. A split over many parts leaves more partials
 // per query tile than the one CU of the last part to arrive can load in good time (64 KB per part
 // at ~64 bytes a clock; parts waiting for each other could deadlock): here every wave loads one
-// 16-byte chunk per lane of up to 16 parts at once, so a tile's partials are spread over 16 waves
-// and all of them are in flight together. Grid (query tile x wave, 32 dims), 4 waves of one chunk
+// 16-byte chunk per lane of up to 16 parts at once, so a tile's partials are spread over 64 waves
+// (16 for each of its column blocks) and all of them are in flight together. Grid (query tile x wave, 32 dims), 4 waves of one chunk
 // each. Parts are merged in part order, 16 at a time (max first, then 2^(m_p - max)-weighted
 // sums), so the result is fixed. GATED (q8_0 caches in F16 precision): when the launch that
 // converted the rows flagged a scale, the whole call is recomputed exactly from the cache.
@@ -1946,7 +1948,10 @@ int required_parts(long long wgs, int keys, int slots) {
 // 22.5 (16); 45 after 1500 24.9 / 18.0 (4) / 17.9 (6); 90 after 6000 74 / 27.2 (8) / 25.5 (10);
 // 90 after 3000 42 / 22.4 (6) / 24.1; 150 after 3000 42 / 23.5 (6) / 28.2; 400 after 3000 45 /
 // 34.9 (2) / 46.3. Short keys are left whole: 60 after 450 (8 tiles) 13.6 unsplit, 15.0 in 4
-// parts; 150 after 700 (14 tiles) 17.6, 16.6 in 3.
+// parts; 150 after 700 (14 tiles) 17.6, 16.6 in 3. At 16 heads over 8, 8 over 8, 64 over 8, 4 over 1
+// and 16 over 4 (20 tokens after 1500, 45 after 5000; f16, q8_0 and f32 caches) factors of 0.7 and
+// 1.4 times these give 0.93 to 1.15 of the time; only in prefill_split_kernel at 16 over 4, 20 after
+// 1500, where 22 parts of 48 stages are uneven (20.5 us), do 24 even ones win (17.3).
 KeySplit split_two_step(double f, long long wgs, int tiles, int slots, int most) {
     const double parts = std::min(f * std::sqrt((double)tiles / wgs) + 0.5,
                                   (double)std::min<long long>(slots / wgs, most));

@@ -133,8 +133,8 @@ struct QkvArgs {
 };
 
 // Row gr of T * (hq + 2 hkv): within a token, first the hq query heads, then the hkv key heads,
-// then the hkv value heads (the reference's order, qkv.metal:59-61). Wave w takes rows
-// 4 w .. 4 w + 3.
+// then the hkv value heads (the reference's order, qkv.metal:59-61). Wave w takes the RPW rows from
+// RPW w on.
 template <int KV, int RPW>
 __global__ void __launch_bounds__(64 * kWavesPerWg) qk_norm_rope_store_kernel(QkvArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t s_stage[kWavesPerWg][KV == BRASA_KV_Q8_0 ? kQ8Row : 4];
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(64 * kWavesPerWg) qk_norm_rope_store_kernel(Qk
     float* dst[RPW];
     size_t crow[RPW];
     int kind[RPW];  // 0 q, 1 k, 2 v, 3 past the last row
-    // every load of the four rows first
+    // every load of the wave's rows first
 #pragma unroll
     for (int j = 0; j < RPW; ++j) {
         const int gr = gr0 + j;

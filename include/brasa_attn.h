@@ -134,7 +134,7 @@ int brasa_dequantize_kv_q8(const void* src, float* dst, size_t rows, void* strea
  * brasa_decode_partials_len(hq, pos0 + 1). Requires tokens == 1, dim == 128 and
  * hq / hkv in {1, 2, 4, 8} (BRASA_ERR_UNSUPPORTED otherwise, where the reference panics).
  * The result bits depend only on q, the cache rows and lk: the launch layout is a function of
- * lk and the head counts (no tuning knob), and the split merge runs in a fixed order, as the
+ * lk, the head counts and the cache type (no tuning knob), and the split merge runs in a fixed order, as the
  * reference requires of every launch width (crates/kernels/tests/launch.rs:119-168). The
  * exception is a stream without a counter slot (more than 64 streams in use on the device),
  * which decodes with one split per sequence: the same result to the decode tolerance, slower.
@@ -178,11 +178,11 @@ int brasa_decode_attention(const float* q, const void* k, const void* v, float* 
  * Ragged batched decode (no counterpart in the reference, which decodes one sequence per call,
  * lib.rs:1110-1164; a caller batching sequences, e.g. a serving scheduler over session.rs:240-245,
  * would otherwise issue one call per sequence). One launch of the split kernel (the split merge
- * runs inside it) covers up to 64 sequences (more: one launch per 64): sequence i has one query q[i] (q: [n, hq, 128] f32), its own layer
- * caches k[i] / v[i] (HOST arrays of device pointers, same layout as decode_attention_lanes) and
- * lk[i] >= 1 keys (HOST array). o: [n, hq, 128] in o_dtype. Each sequence's result agrees with
+ * runs inside it) covers up to 64 sequences (more: one launch per 64): sequence i has one query q[i]
+ * (q: [n, hq, 128] f32), its own layer caches k[i] / v[i] (HOST arrays of device pointers, same
+ * layout as decode_attention_lanes) and lk[i] >= 1 keys (HOST array). o: [n, hq, 128] in o_dtype. Each sequence's result agrees with
  * brasa_decode_attention_lanes on it alone to the decode tolerance, not bit for bit: a launch
- * cuts every sequence into splits of one length chosen from the batch's total keys, so the split
+ * cuts every sequence into splits of one length chosen from all of the batch's lengths, so the split
  * boundaries (and the f32 rounding of the merge) differ from the single-sequence call's. A
  * single-sequence call's result depends only on its inputs and lk. Scratch: partials_len >=
  * brasa_decode_batch_partials_len(hq, lk, n) floats. Requires dim == 128 and a GQA group in
@@ -206,7 +206,8 @@ int brasa_decode_attention_batch(const float* q, const void* const* k, const voi
  * that would fill at most half of the GPU with long key ranges per query tile (a short chunk
  * after a long cached prefix, e.g. 512 tokens at pos0 16384) splits each tile's keys over several
  * workgroups (up to 32); their partials go to a workspace (68 KB per part and query tile, at
- * most 512 of them), merged in the same launch or, with few query tiles, by a launch of its own. With a q8_0
+ * most 512 of them), merged in the same launch or, with few query tiles or many parts, by a launch
+ * of its own. With a q8_0
  * cache and BRASA_PREFILL_F16, the rows read (ceil64(pos0 + tokens) positions) are first
  * dequantised to f16 (each value f16(code * scale)) into the workspace (512 B per row of K and
  * V), and the f16 kernels run on it; small calls and calls of one query tile convert the same
