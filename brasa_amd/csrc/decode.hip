@@ -538,8 +538,8 @@ __device__ __forceinline__ void finish_split(const DecodeArgs<NS>& a, const SeqD
 // by ds_read_tr16_b64), Q HBM -> LDS. Every vector-memory instruction of the block loop is inline
 // asm. A wave keeps one block in flight: block i + 1 is issued into the other ring slot once block
 // i has landed; two from the start only lengthen the memory system's queues, and every wave's
-// first block lands later (16K keys: 16.1 us a layer with one, 16.45 with two; 1000 keys 7.25,
-// 7.9). Four heads per workgroup, the layout of large batches, keep two (59.0 us against 59.35 for
+// first block lands later (1000 keys 7.25 us a layer with one, 7.9 with two; at 16K 16.15 and 16.30
+// on one box, about what runs differ). Four heads per workgroup, the layout of large batches, keep two (59.0 us against 59.35 for
 // 8 sequences of 1024 to 16384 keys). The wait names the K registers it guards as operands, so no
 // use of them can be scheduled above it.
 // Softmax: columns c < G hold the hi halves of the split Q / P operands, the partner columns
