@@ -470,11 +470,20 @@ TWO_STEP_HEADS = [(8, 8, KvType.F16, "F16", 100, 1500), (8, 8, KvType.Q8_0, "F16
                   (4, 1, KvType.Q8_0, "F16", 383, 0)]
 
 
-@pytest.mark.parametrize("hq,hkv,kv,precision,tokens,pos0",
-                         [(HQ, HKV, *c) for c in TWO_STEP] + TWO_STEP_HEADS)
-def test_flash_key_split_own_launch(hq, hkv, kv, precision, tokens, pos0):
+@pytest.mark.parametrize("kv,precision,tokens,pos0", TWO_STEP)
+def test_flash_key_split_own_launch(kv, precision, tokens, pos0):
     """Key splits merged by prefill_merge_kernel, at the bars of the unsplit kernels; repeat calls
     give equal bits (the parts merge in a fixed order), and garbage past the last key is masked."""
+    check_own_launch(HQ, HKV, kv, precision, tokens, pos0)
+
+
+@pytest.mark.parametrize("hq,hkv,kv,precision,tokens,pos0", TWO_STEP_HEADS)
+def test_flash_key_split_own_launch_heads(hq, hkv, kv, precision, tokens, pos0):
+    """The same at the other GQA groups and at more query tiles."""
+    check_own_launch(hq, hkv, kv, precision, tokens, pos0)
+
+
+def check_own_launch(hq, hkv, kv, precision, tokens, pos0):
     prec = PrefillPrecision[precision]
     synchronize()
     assert lib().brasa_release_workspaces() == 0
